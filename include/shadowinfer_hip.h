@@ -81,6 +81,10 @@ int si_check_bf16_convert(unsigned long long* counts, si_stream_t stream);
 void si_tune_gemm_plan(int kind, int splits);
 void si_tune_attn_offset64(int on);
 
+/* Test and sweep override of the split of a short attention over workgroups:
+ * 0 (the start value) by size, -1 never, n > 0 n parts where it applies. */
+void si_tune_attn_parts(int parts);
+
 /* Thread-local text of the last failure (empty string if none). Replaces the
  * TORCH_CHECK messages of shadowinfer/kernels/cpp/quantize_int4.cu:176-177. */
 const char* si_last_error(void);
@@ -299,6 +303,22 @@ int si_attn_packed_fwd_built(const void* q, int q_dtype, int64_t B, int64_t H, i
                              const void* const* buckets, int scale_dtype, int64_t S_kv,
                              int64_t group, float sm_scale, void* out, int out_dtype,
                              int token_major, si_stream_t stream);
+
+/* si_attn_packed_fwd_built with a workspace for calls whose query blocks
+ * leave most CUs idle (few queries, or few heads): their keys are then split
+ * over workgroups, whose partial results pass through the workspace.
+ * si_attn_parts_bytes is what a call of that shape takes (0 for most); with a
+ * smaller or NULL workspace (16-byte aligned) the keys are not split. A split
+ * call rounds the probabilities at other running maxima: split == 0 keeps one
+ * kernel, so the same bits for a query row, at every size. */
+size_t si_attn_parts_bytes(int64_t B, int64_t H, int64_t S_q, int64_t D, int64_t S_kv,
+                           int scale_dtype);
+int si_attn_packed_fwd_parts(const void* q, int q_dtype, int64_t B, int64_t H, int64_t S_q,
+                             int64_t D, const void* lists, size_t lists_bytes,
+                             const void* const* buckets, int scale_dtype, int64_t S_kv,
+                             int64_t group, float sm_scale, void* out, int out_dtype,
+                             int token_major, int split, void* workspace,
+                             size_t workspace_bytes, si_stream_t stream);
 
 /* ---------------------------------------------------------------------- */
 /* Quantizer                                                               */

@@ -22,6 +22,7 @@
 // fp32 online softmax; fp16 entries of the cache are exact in fp16, int8/int4
 // values q*s are rounded once to fp16, and P is rounded to fp16 for the P.V
 // MFMAs (its row sum adds the same fp16 values).
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -265,7 +266,8 @@ __device__ __forceinline__ float halves_sum(float v) {
 }
 
 // ---------------------------------------------------------------------------
-// The three parts of one 64-key tile for the 32 queries of a wave.
+// The three parts of one tile of KB 32-key blocks (64 keys) for the 32 queries
+// of a wave.
 //
 // tile_qk: S^T = K Q^T - m on v_mfma_f32_32x32x16_f16. The accumulators start
 // at -m_run (0 before the first tile), so the MFMAs return the scores already
@@ -274,25 +276,27 @@ __device__ __forceinline__ float halves_sum(float v) {
 // MFMAs of k-step ks run. Raises the wave priority (the caller lowers it after
 // the tile's last P.V MFMA): when both waves of a SIMD have instructions
 // ready, the one feeding the matrix core issues first.
-template <int D>
+template <int D, int KB = 2>
 __device__ __forceinline__ void tile_qk(const _Float16 (*Ks)[D + KPAD], const v8h* qf, int col,
-                                        int grp, const v16f& cinit, v16f (&sacc)[2]) {
+                                        int grp, const v16f& cinit, v16f (&sacc)[KB]) {
   constexpr int KS = D / 16;
-  v8h ka[2][2];
+  v8h ka[2][KB];
   auto load_k = [&](int ks, v8h* a) __attribute__((always_inline)) {
-    a[0] = *reinterpret_cast<const v8h*>(&Ks[col][ks * 16 + 8 * grp]);
-    a[1] = *reinterpret_cast<const v8h*>(&Ks[32 + col][ks * 16 + 8 * grp]);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      a[kb] = *reinterpret_cast<const v8h*>(&Ks[32 * kb + col][ks * 16 + 8 * grp]);
   };
   load_k(0, ka[0]);
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     if (ks + 1 < KS) load_k(ks + 1, ka[(ks + 1) & 1]);
-    sacc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks & 1][0], qf[ks], ks == 0 ? cinit : sacc[0], 0, 0, 0);
-    sacc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks & 1][1], qf[ks], ks == 0 ? cinit : sacc[1], 0, 0, 0);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks & 1][kb], qf[ks], ks == 0 ? cinit : sacc[kb], 0, 0, 0);
     if (ks + 1 < KS) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the two reads of ks+1
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // then the two MFMAs of ks
+      __builtin_amdgcn_sched_group_barrier(0x100, KB, 0);  // the reads of ks+1
+      __builtin_amdgcn_sched_group_barrier(0x008, KB, 0);  // then the MFMAs of ks
     }
   }
 }
@@ -302,16 +306,19 @@ __device__ __forceinline__ void tile_qk(const _Float16 (*Ks)[D + KPAD], const v8
 // then carry K to about 22 bits instead of fp16's 11. With fp32 K/V holding
 // outlier channels, K's fp16 rounding is most of the output's error (a model
 // of the kernel's roundings: relL2 8.8e-4 with it, 4.4e-4 without).
-template <int D>
+template <int D, int KB = 2>
 __device__ __forceinline__ void tile_qk_lo(const _Float16 (*Kl)[D + KPAD], const v8h* qf, int col,
-                                           int grp, v16f (&sacc)[2]) {
+                                           int grp, v16f (&sacc)[KB]) {
   constexpr int KS = D / 16;
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    const v8h a0 = *reinterpret_cast<const v8h*>(&Kl[col][ks * 16 + 8 * grp]);
-    const v8h a1 = *reinterpret_cast<const v8h*>(&Kl[32 + col][ks * 16 + 8 * grp]);
-    sacc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, qf[ks], sacc[0], 0, 0, 0);
-    sacc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qf[ks], sacc[1], 0, 0, 0);
+    v8h a[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      a[kb] = *reinterpret_cast<const v8h*>(&Kl[32 * kb + col][ks * 16 + 8 * grp]);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kb], qf[ks], sacc[kb], 0, 0, 0);
   }
 }
 
@@ -321,22 +328,22 @@ __device__ __forceinline__ void tile_qk_lo(const _Float16 (*Kl)[D + KPAD], const
 // and always at the first tile, so the output rescale is rare. P = 2^(s - m)
 // as fp16 pairs (the B operand of the P.V MFMAs); the row sum adds the same
 // fp16 values in fp32 (v_dot2_f32_f16 with {1, 1}).
-template <int D>
-__device__ __forceinline__ void tile_softmax(v16f (&sacc)[2], int nv, int grp, float& m_run,
+template <int D, int KB = 2>
+__device__ __forceinline__ void tile_softmax(v16f (&sacc)[KB], int nv, int grp, float& m_run,
                                              v16f& cinit, float& l_run, v16f* o,
-                                             uint32_t (&pw)[16]) {
+                                             uint32_t (&pw)[8 * KB]) {
   constexpr int DB = D / 32;
   const float c0 = m_run == -INFINITY ? 0.0f : -m_run;
-  if (nv < BN) {
+  if (nv < 32 * KB) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (kb * 32 + 8 * (r >> 2) + 4 * grp + (r & 3) >= nv) sacc[kb][r] = -INFINITY;
   }
   float tm[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+  for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
     for (int r = 0; r < 16; ++r) tm[r & 3] = fmaxf(tm[r & 3], sacc[kb][r]);
   float tmax = fmaxf(fmaxf(tm[0], tm[1]), fmaxf(tm[2], tm[3]));
@@ -352,7 +359,7 @@ __device__ __forceinline__ void tile_softmax(v16f (&sacc)[2], int nv, int grp, f
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) sacc[kb][r] -= delta;
     m_run = m_new;
@@ -360,7 +367,7 @@ __device__ __forceinline__ void tile_softmax(v16f (&sacc)[2], int nv, int grp, f
     for (int r = 0; r < 16; ++r) cinit[r] = m_new == -INFINITY ? 0.0f : -m_new;
   }
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+  for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       // v_exp_f32: arguments are <= 8 here; results below 2^-126 flush to 0
@@ -371,7 +378,7 @@ __device__ __forceinline__ void tile_softmax(v16f (&sacc)[2], int nv, int grp, f
   float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   const h2 ones = {(_Float16)1.0f, (_Float16)1.0f};
 #pragma unroll
-  for (int w = 0; w < 16; ++w) ps[w & 3] = __builtin_amdgcn_fdot2(as_h2(pw[w]), ones, ps[w & 3], false);
+  for (int w = 0; w < 8 * KB; ++w) ps[w & 3] = __builtin_amdgcn_fdot2(as_h2(pw[w]), ones, ps[w & 3], false);
   l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);  // this half's keys; halves added at the end
 }
 
@@ -384,9 +391,9 @@ __device__ __forceinline__ void tile_softmax(v16f (&sacc)[2], int nv, int grp, f
 // addresses key k0 + i/4 at dims base + 4*(i%4), and lane r receives dim
 // base + r of keys k0 .. k0+3. V^T fragments stream two (chunk, row block)
 // steps ahead of their MFMA.
-template <int D>
+template <int D, int KB = 2>
 __device__ __forceinline__ void tile_pv(const _Float16 (*Vs)[AttnCfg<D>::VROW],
-                                        const uint32_t (&pw)[16], int col, int grp, v16f* o) {
+                                        const uint32_t (&pw)[8 * KB], int col, int grp, v16f* o) {
   constexpr int DB = D / 32;
   const int li = col & 15;       // lane within its 16-lane group
   const int half = col >> 4;     // dims 0..15 or 16..31 of a 32-dim block
@@ -398,7 +405,7 @@ __device__ __forceinline__ void tile_pv(const _Float16 (*Vs)[AttnCfg<D>::VROW],
         v4h, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(vp + 8 * AttnCfg<D>::VROW)));
     return v8h{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   };
-  constexpr int NV = 4 * DB;
+  constexpr int NV = 2 * KB * DB;
   v8h va[3];
   va[0] = load_v(0);
   va[1] = load_v(1);
@@ -1003,6 +1010,420 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
                  os.s, O, odt);
 }
 
+// ---------------------------------------------------------------------------
+// The same attention for few query blocks: a wave per 32-key half tile.
+//
+// attn_packed_fwd gives a block 256 queries and all keys of a head, so a call
+// with ceil(S_q / 256) * H * B < 256 leaves CUs idle (32 queries, 32 heads, 4096
+// keys: 32 blocks of which one wave in eight holds queries, 112 us for 40 MB of
+// packed rows). Here a block of 8 waves owns 32 queries of one (b, h) and one of
+// nch interleaved parts of the head's keys; wave w of part c takes the half
+// tiles 8 c + w + 8 nch i, decodes them into LDS of its own (so no barrier stands in
+// the loop) and keeps its own (m, l, O). The waves are added in LDS at the end
+// and, with nch > 1, the parts by attn_combine. Every wave decodes its keys
+// alone, which costs about three times the VALU work per query of the
+// 256-query blocks: attn_parts decides where that pays.
+//
+// Rows: LPR = D / 8 lanes hold 8 dims each of one key, and lane group j of
+// 64 / LPR takes keys RPL * j .. + RPL - 1 of the half tile, so every load
+// instruction reads whole bucket rows. The rows of the wave's next half tile are
+// loaded while the current one is multiplied.
+// ---------------------------------------------------------------------------
+constexpr int HN = 32;  // keys per half tile
+
+template <int D>
+struct ShortCfg {
+  static constexpr int NW = 8;              // waves per block
+  static constexpr int LPR = D / 8;         // lanes per key row
+  static constexpr int RPL = HN * LPR / 64; // key rows per lane
+  static constexpr int KB = HN * (D + KPAD) * 2;           // bytes of a wave's K rows
+  static constexpr int VB = HN * AttnCfg<D>::VROW * 2;     // bytes of a wave's V rows
+  static constexpr int BUF = KB + VB;
+  static constexpr int OP = D + 4;          // floats per staged output row
+  static constexpr int DPT = D * 32 / 512;  // output values per thread of a 32-row result
+};
+
+// Orders this wave's own LDS accesses (the hardware runs them in order; the
+// compiler must not move them across).
+__device__ __forceinline__ void wave_lds_order() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_wave_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// Final scaling of DPT consecutive output values: evicted keys join the
+// denominator (score 0, value 0), then the division and the rounding to odt.
+template <int DPT>
+__device__ __forceinline__ void short_store(float (&acc)[DPT], float M, float L, int n_ev, void* O,
+                                            int64_t at, int odt) {
+  if (n_ev > 0) {
+    const float mf = fmaxf(M, 0.0f);
+    const float a = exp2f(M - mf);
+    L = L * a + (float)n_ev * exp2f(-mf);
+#pragma unroll
+    for (int i = 0; i < DPT; ++i) acc[i] *= a;
+  }
+  const float inv = 1.0f / L;
+  if (odt == SI_DT_F32) {
+    float* p = reinterpret_cast<float*>(O) + at;
+#pragma unroll
+    for (int i = 0; i < DPT; i += 4)
+      *reinterpret_cast<float4*>(p + i) = make_float4(acc[i] * inv, acc[i + 1] * inv,
+                                                      acc[i + 2] * inv, acc[i + 3] * inv);
+  } else {
+    const bool bf = odt == SI_DT_BF16;
+    uint32_t w[DPT / 2];
+#pragma unroll
+    for (int i = 0; i < DPT / 2; ++i) {
+      const float x = acc[2 * i] * inv, y = acc[2 * i + 1] * inv;
+      w[i] = (bf ? f32_to_bf16_bits(x) : f32_to_f16_bits(x)) |
+             ((bf ? f32_to_bf16_bits(y) : f32_to_f16_bits(y)) << 16);
+    }
+    uint16_t* p = reinterpret_cast<uint16_t*>(O) + at;
+#pragma unroll
+    for (int i = 0; i < DPT / 2; i += 2)
+      *reinterpret_cast<uint2*>(p + 2 * i) = make_uint2(w[i], w[i + 1]);
+  }
+}
+
+// Requires int4 groups of 8 * n dims. O32: 32-bit row offsets, as in
+// attn_packed_fwd.
+template <int D, int SDT, bool O32>
+__global__ __launch_bounds__(512) void attn_packed_short(
+    const uint16_t* __restrict__ Q, int qdt, int64_t B, int64_t H, int64_t Sq, int64_t cap,
+    const int32_t* __restrict__ counts, const int32_t* __restrict__ lists, Buckets bk, int64_t g,
+    float scale_log2, void* __restrict__ O, int odt, OutStrides os, int nq, int nch,
+    float* __restrict__ part, float* __restrict__ part_ml) {
+  using C = ShortCfg<D>;
+  constexpr int KS = D / 16, DB = D / 32, LPR = C::LPR, RPL = C::RPL;
+  constexpr bool KLO = SDT == SI_DT_F32;
+  __shared__ __attribute__((aligned(16))) uint8_t bufs[C::NW * C::BUF];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, grp = lane >> 5;
+  // Parts and query groups of one (b, h) on one XCD, as in attn_packed_fwd.
+  const int w_id = xcd_order((int)blockIdx.x, (int)gridDim.x);
+  const int unit = w_id / nch, ch = w_id % nch;  // unit: (b * H + h) * nq + query group
+  const int bh = unit / nq;
+  const int64_t h = bh % (int)H, b = bh / (int)H;
+  const int64_t m0 = (int64_t)(unit % nq) * 32;
+
+  const int32_t* lh = lists + h * cap;
+  const int row0 = lane / LPR * RPL, d0 = lane % LPR * 8;
+  const int first = C::NW * ch + wave, step = C::NW * nch;
+  const int last_list = (int)(cap / HN) - 1;  // of the head's list, whatever the counts are
+  // Slots of this lane's rows of half tile u.
+  auto slots = [&](int64_t u, int (&sl)[RPL]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < RPL; i += 4) {
+      const int4 v = *reinterpret_cast<const int4*>(lh + u * HN + row0 + i);
+      sl[i] = v.x; sl[i + 1] = v.y; sl[i + 2] = v.z; sl[i + 3] = v.w;
+    }
+  };
+  // The first half tile's slots do not wait for the counts.
+  int sl[RPL];
+  slots(min(first, last_list), sl);
+  v8h qf[KS];
+  if (qdt == SI_DT_BF16) load_q<D, SI_DT_BF16>(Q, b, H, h, Sq, m0 + col, grp, scale_log2, qf);
+  else load_q<D, SI_DT_F16>(Q, b, H, h, Sq, m0 + col, grp, scale_log2, qf);
+  const int32_t* cnt = counts + h * 8;
+
+  uint8_t* buf = bufs + wave * C::BUF;
+  auto Kt = reinterpret_cast<_Float16 (*)[D + KPAD]>(buf);
+  auto Vt = reinterpret_cast<_Float16 (*)[AttnCfg<D>::VROW]>(buf + C::KB);
+  auto Kl = reinterpret_cast<_Float16 (*)[D + KPAD]>(buf + C::KB);  // low parts of K, before V
+  static_assert(C::KB <= C::VB, "the low parts fit V's rows");
+
+  constexpr uint32_t SS = SDT == SI_DT_F32 ? 4 : 2;  // scale bytes
+  const uint32_t ngrp = (uint32_t)((int)D / (int)g), my_grp = (uint32_t)(d0 / (int)g);
+
+  v16f o[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[i][r] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;
+  v16f cinit = {};
+
+  int u = first;     // next half tile of this wave
+  int hs = 0;        // first half tile of the phase
+  // To this wave's first half tile past the phase's last tile, whose second
+  // half may be empty.
+  auto skip_to_phase_end = [&]() __attribute__((always_inline)) {
+    if (u >= hs) return;
+    while (u < hs) u += step;
+    slots(min(u, last_list), sl);
+  };
+  auto run_phase = [&](auto PC) __attribute__((always_inline)) {
+    constexpr int P = decltype(PC)::value;
+    constexpr int WB = P == SI_PREC_FP32 ? 32 : P == SI_PREC_FP16 ? 16 : P == SI_PREC_INT8 ? 8 : 4;
+    constexpr bool INT = P == SI_PREC_INT8 || P == SI_PREC_INT4;
+    constexpr int W = WB / 4;  // 32-bit words of 8 dims
+    const int n = cnt[P];
+    const int he = hs + (n + HN - 1) / HN;
+    const int n_end = n + hs * HN;  // list position after the phase's last key
+    hs += (n + BN - 1) / BN * (BN / HN);
+    if (u >= he) {
+      skip_to_phase_end();
+      return;
+    }
+    auto base = [&](int j) __attribute__((always_inline)) {
+      return reinterpret_cast<const char*>(bk.p[4 * P + j]);
+    };
+    using off_t = std::conditional_t<O32, uint32_t, uint64_t>;
+    auto mul = [&](uint32_t x, off_t y) __attribute__((always_inline)) -> off_t {
+      if constexpr (O32) return __umul24(x, y);
+      else return x * y;
+    };
+    const off_t st = (off_t)(B * D) * WB / 8, c0 = (off_t)(b * D + d0) * WB / 8;
+    const off_t sst = (off_t)B * SS * (P == SI_PREC_INT4 ? ngrp : 1u);
+    const off_t sc0 = (P == SI_PREC_INT4 ? (off_t)b * ngrp + my_grp : (off_t)b) * SS;
+    // fp32 rows are read in two steps (K, then V): 32 bytes of each of K and V
+    // per lane and row would not fit the registers.
+    constexpr bool BOTH = P != SI_PREC_FP32;
+    uint32_t rk[RPL][W], rv[BOTH ? RPL : 1][W], skb[RPL], svb[RPL], us[RPL];
+    auto load_rows = [&](int uu) __attribute__((always_inline)) {
+      const int nv = n_end - uu * HN;
+      // Keys past the phase's last read row 0 of the (non-empty) bucket: their
+      // list entries are not written; their scores are masked.
+#pragma unroll
+      for (int i = 0; i < RPL; ++i) {
+        us[i] = (uint32_t)(row0 + i < nv ? sl[i] : 0);
+        if constexpr (O32) __builtin_assume(us[i] < (1u << 23));
+      }
+#pragma unroll
+      for (int i = 0; i < RPL; ++i) {
+        const off_t off = mul(us[i], st) + c0;
+        if constexpr (P == SI_PREC_FP32) {
+          load_raw<16>(base(0) + off, rk[i]);
+          load_raw<16>(base(0) + off + 16, rk[i] + 4);
+        } else {
+          load_raw<WB>(base(0) + off, rk[i]);
+          load_raw<WB>(base(1) + off, rv[i]);
+        }
+        if constexpr (INT) {
+          const off_t so = mul(us[i], sst) + sc0;
+          load_raw<SS>(base(2) + so, &skb[i]);
+          load_raw<SS>(base(3) + so, &svb[i]);
+        }
+      }
+    };
+    // Eight integer codes of row i as fp16 pairs.
+    auto codes = [&](const uint32_t* r, uint32_t (&w)[4]) __attribute__((always_inline)) {
+      if constexpr (P == SI_PREC_INT8) {
+        i8x4_to_h(r[0], w[0], w[1]);
+        i8x4_to_h(r[1], w[2], w[3]);
+      } else {
+        i4x4_to_h(r[0], w[0], w[1]);
+        i4x4_to_h(r[0] >> 16, w[2], w[3]);
+      }
+    };
+    auto all_exact = [&](const uint32_t (&sb)[RPL]) __attribute__((always_inline)) {
+      int fast = 1;
+#pragma unroll
+      for (int i = 0; i < RPL; ++i)
+        fast &= (int)h_exact<SDT, P == SI_PREC_INT8>(sb[i], scale_from_bits<SDT>(sb[i]));
+      return __builtin_amdgcn_ballot_w64(fast == 0) == 0;
+    };
+    // Codes times scale rounded once to fp16: a packed fp16 multiply where that
+    // rounds like the fp32 product for every row of the wave (see decode_tile),
+    // else through fp32.
+    auto decode = [&](const uint32_t (*r)[W], const uint32_t (&sb)[RPL], auto&& put)
+        __attribute__((always_inline)) {
+      const bool fast = all_exact(sb);
+#pragma unroll
+      for (int i = 0; i < RPL; ++i) {
+        uint32_t w[4];
+        codes(r[i], w);
+        const float s = scale_from_bits<SDT>(sb[i]);
+        if (fast) {
+          const h2 s2 = scale_h2<SDT>(sb[i], s);
+#pragma unroll
+          for (int x = 0; x < 4; ++x) w[x] = as_u32(as_h2(w[x]) * s2);
+        } else {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const h2 a = as_h2(w[x]);
+            w[x] = pack_h2((_Float16)((float)a[0] * s), (_Float16)((float)a[1] * s));
+          }
+        }
+        put(row0 + i, make_uint4(w[0], w[1], w[2], w[3]));
+      }
+    };
+    auto f8 = [](const float* f) __attribute__((always_inline)) {
+      return make_uint4(pack_h2((_Float16)f[0], (_Float16)f[1]), pack_h2((_Float16)f[2], (_Float16)f[3]),
+                        pack_h2((_Float16)f[4], (_Float16)f[5]), pack_h2((_Float16)f[6], (_Float16)f[7]));
+    };
+    auto put_k = [&](int r, uint4 w) __attribute__((always_inline)) { *reinterpret_cast<uint4*>(&Kt[r][d0]) = w; };
+    auto put_l = [&](int r, uint4 w) __attribute__((always_inline)) { *reinterpret_cast<uint4*>(&Kl[r][d0]) = w; };
+    auto put_v = [&](int r, uint4 w) __attribute__((always_inline)) { *reinterpret_cast<uint4*>(&Vt[r][d0]) = w; };
+
+    load_rows(u);
+    while (true) {
+      const int nx = u + step;
+      const int nv = __builtin_amdgcn_readfirstlane(min(HN, n_end - u * HN));
+      slots(min(nx, last_list), sl);  // also when nx belongs to the next phase
+      // K rows (and their low parts with KLO), V rows
+#pragma unroll
+      for (int i = 0; i < RPL; ++i) {
+        if constexpr (P == SI_PREC_FP16) {
+          put_k(row0 + i, make_uint4(rk[i][0], rk[i][1], rk[i][2], rk[i][3]));
+          put_v(row0 + i, make_uint4(rv[i][0], rv[i][1], rv[i][2], rv[i][3]));
+        } else if constexpr (P == SI_PREC_FP32 || KLO) {
+          float f[8], lo[8];
+          if constexpr (P == SI_PREC_FP32) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = __builtin_bit_cast(float, rk[i][e]);
+          } else {
+            uint32_t w[4];
+            codes(rk[i], w);
+            const float s = scale_from_bits<SDT>(skb[i]);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const h2 a = as_h2(w[x]);
+              f[2 * x] = (float)a[0] * s;
+              f[2 * x + 1] = (float)a[1] * s;
+            }
+          }
+          put_k(row0 + i, f8(f));
+          if constexpr (KLO) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) lo[e] = f[e] - (float)(_Float16)f[e];
+            put_l(row0 + i, f8(lo));
+          }
+        }
+      }
+      if constexpr (INT && !KLO) {
+        decode(rk, skb, put_k);
+        decode(rv, svb, put_v);
+      }
+      if constexpr (P == SI_PREC_FP32) {  // V, into the registers of K
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) {
+          const off_t off = mul(us[i], st) + c0;
+          load_raw<16>(base(1) + off, rk[i]);
+          load_raw<16>(base(1) + off + 16, rk[i] + 4);
+        }
+      }
+      wave_lds_order();
+      // Rows of the next half tile, unless this one's V is still in registers.
+      constexpr bool LATE_V = P == SI_PREC_FP32 || (INT && KLO);
+      if constexpr (!LATE_V)
+        if (nx < he) load_rows(nx);
+      v16f sacc[1];
+      uint32_t pw[8];
+      tile_qk<D, 1>(Kt, qf, col, grp, cinit, sacc);
+      if constexpr (KLO && P != SI_PREC_FP16) tile_qk_lo<D, 1>(Kl, qf, col, grp, sacc);
+      tile_softmax<D, 1>(sacc, nv, grp, m_run, cinit, l_run, o, pw);
+      if constexpr (LATE_V) {
+        wave_lds_order();
+        if constexpr (P == SI_PREC_FP32) {
+#pragma unroll
+          for (int i = 0; i < RPL; ++i) {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = __builtin_bit_cast(float, rk[i][e]);
+            put_v(row0 + i, f8(f));
+          }
+        } else {
+          decode(rv, svb, put_v);
+        }
+        wave_lds_order();
+        if (nx < he) load_rows(nx);
+      }
+      tile_pv<D, 1>(Vt, pw, col, grp, o);
+      __builtin_amdgcn_s_setprio(0);
+      wave_lds_order();
+      u = nx;
+      if (u >= he) break;
+    }
+    skip_to_phase_end();
+  };
+  run_phase(std::integral_constant<int, SI_PREC_FP32>{});
+  run_phase(std::integral_constant<int, SI_PREC_FP16>{});
+  run_phase(std::integral_constant<int, SI_PREC_INT8>{});
+  run_phase(std::integral_constant<int, SI_PREC_INT4>{});
+
+  // Each wave's O rows and (m, l) into its own buffer, then the 8 are added.
+  {
+    float* so = reinterpret_cast<float*>(buf);
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(so + col * C::OP + db * 32 + 8 * i + 4 * grp) =
+            make_float4(o[db][4 * i], o[db][4 * i + 1], o[db][4 * i + 2], o[db][4 * i + 3]);
+    l_run = halves_sum(l_run);
+    if (grp == 0) *reinterpret_cast<float2*>(so + 32 * C::OP + 2 * col) = make_float2(m_run, l_run);
+  }
+  static_assert((32 * C::OP + 64) * 4 <= C::BUF, "staged rows fit a wave's buffer");
+  __syncthreads();
+  const int q = tid / 16, d = tid % 16 * C::DPT;
+  float mw[C::NW], M = -INFINITY, L = 0.0f;
+#pragma unroll
+  for (int w = 0; w < C::NW; ++w) {
+    mw[w] = reinterpret_cast<const float*>(bufs + w * C::BUF)[32 * C::OP + 2 * q];
+    M = fmaxf(M, mw[w]);
+  }
+  float acc[C::DPT] = {};
+#pragma unroll
+  for (int w = 0; w < C::NW; ++w) {
+    const float* sw = reinterpret_cast<const float*>(bufs + w * C::BUF);
+    const float a = mw[w] == -INFINITY ? 0.0f : exp2f(mw[w] - M);  // -inf: no tile
+    L += a * sw[32 * C::OP + 2 * q + 1];
+#pragma unroll
+    for (int i = 0; i < C::DPT; i += 4) {
+      const float4 v = *reinterpret_cast<const float4*>(sw + q * C::OP + d + i);
+      acc[i] += a * v.x; acc[i + 1] += a * v.y; acc[i + 2] += a * v.z; acc[i + 3] += a * v.w;
+    }
+  }
+  if (nch == 1) {
+    if (m0 + q < Sq)
+      short_store<C::DPT>(acc, M, L, cnt[4], O, b * os.b + h * os.h + (m0 + q) * os.s + d, odt);
+    return;
+  }
+  if (m0 + q >= Sq) return;
+  const int64_t pr = ((int64_t)unit * nch + ch) * 32 + q;
+#pragma unroll
+  for (int i = 0; i < C::DPT; i += 4)
+    *reinterpret_cast<float4*>(part + pr * D + d + i) = make_float4(acc[i], acc[i + 1], acc[i + 2], acc[i + 3]);
+  if (tid % 16 == 0) *reinterpret_cast<float2*>(part_ml + 2 * pr) = make_float2(M, L);
+}
+
+// Adds the nch parts of each 32-query unit, 4 queries per one-wave block (a few
+// units must still fill the chip).
+template <int D>
+__global__ __launch_bounds__(64) void attn_combine(const float* __restrict__ part,
+                                                    const float* __restrict__ part_ml, int nch,
+                                                    int nq, int64_t H, int64_t Sq,
+                                                    const int32_t* __restrict__ counts,
+                                                    void* __restrict__ O, int odt, OutStrides os) {
+  constexpr int DPT = ShortCfg<D>::DPT;
+  const int unit = (int)blockIdx.x / 8;
+  const int64_t bh = unit / nq, h = bh % H, b = bh / H;
+  const int q = (int)blockIdx.x % 8 * 4 + threadIdx.x / 16, d = threadIdx.x % 16 * DPT;
+  const int64_t m = (int64_t)(unit % nq) * 32 + q;
+  if (m >= Sq) return;
+  const int64_t r0 = (int64_t)unit * nch * 32 + q;
+  float M = -INFINITY, L = 0.0f;
+  for (int c = 0; c < nch; ++c) M = fmaxf(M, part_ml[2 * (r0 + 32 * c)]);
+  float acc[DPT] = {};
+#pragma unroll 4
+  for (int c = 0; c < nch; ++c) {
+    const float2 ml = *reinterpret_cast<const float2*>(part_ml + 2 * (r0 + 32 * c));
+    const float a = ml.x == -INFINITY ? 0.0f : exp2f(ml.x - M);
+    L += a * ml.y;
+    const float* src = part + (r0 + 32 * c) * D + d;
+#pragma unroll
+    for (int i = 0; i < DPT; i += 4) {
+      const float4 v = *reinterpret_cast<const float4*>(src + i);
+      acc[i] += a * v.x; acc[i + 1] += a * v.y; acc[i + 2] += a * v.z; acc[i + 3] += a * v.w;
+    }
+  }
+  short_store<DPT>(acc, M, L, counts[h * 8 + 4], O, b * os.b + h * os.h + m * os.s + d, odt);
+}
+
 template <int D, int QDT, bool O32>
 void launch_attn_o(int sdt, dim3 grid, hipStream_t st, const uint16_t* q, int64_t B, int64_t H,
                    int64_t Sq, int64_t cap, const int32_t* counts, const int32_t* lists,
@@ -1029,15 +1450,19 @@ std::atomic<int> g_force_offset64{0};
 
 // A bucket holds at most n_max = S_kv * H entries; fp32 rows (B * D * 4 bytes)
 // bound the byte offsets of every bucket and scale buffer.
+// si_tune_attn_offset64 selects the 64-bit addressing at every size, so tests can
+// compare the two paths on small caches.
+bool offsets32(int64_t n_max, int64_t B, int64_t D) {
+  return n_max * B * D * 4 < ((int64_t)1 << 31) && B * D < ((int64_t)1 << 21) &&
+         !g_force_offset64.load(std::memory_order_relaxed);
+}
+
 template <int D, int QDT>
 void launch_attn(int sdt, dim3 grid, hipStream_t st, const uint16_t* q, int64_t B, int64_t H,
                  int64_t Sq, int64_t cap, const int32_t* counts, const int32_t* lists,
                  const Buckets& bk, int64_t g, float scale_log2, void* out, int odt,
                  const OutStrides& os, int64_t n_max) {
-  // si_tune_attn_offset64 selects the 64-bit addressing at every size, so tests can
-  // compare the two paths on small caches.
-  if (n_max * B * D * 4 < ((int64_t)1 << 31) && B * D < ((int64_t)1 << 21) &&
-      !g_force_offset64.load(std::memory_order_relaxed))
+  if (offsets32(n_max, B, D))
     launch_attn_o<D, QDT, true>(sdt, grid, st, q, B, H, Sq, cap, counts, lists, bk, g, scale_log2,
                                 out, odt, os);
   else
@@ -1045,10 +1470,92 @@ void launch_attn(int sdt, dim3 grid, hipStream_t st, const uint16_t* q, int64_t 
                                  out, odt, os);
 }
 
+// Parts of attn_packed_short for a call, 0 for attn_packed_fwd (see run_attn for
+// what the short kernel asks of the buffers). Set by si_tune_attn_parts (tests
+// and sweeps): 0 automatic, -1 never the short kernel, n > 0 that many parts.
+std::atomic<int> g_force_parts{0};
+
+//
+// The rule compares two time estimates (us), fitted on S_kv = 100..8192, H = 4..32:
+// attn_packed_fwd takes 9 + 1.6 per 64-key tile and round of 256 blocks (D = 64:
+// 1.2; 2.0 where its blocks fill over half the chip, as the clock then drops),
+// the short kernel 6 + 2.15 per half tile and wave (D = 64: 1.3) and, with n > 1
+// parts, 3.5 for the second launch and the partial rows at 3 TB/s; caches of fp32
+// inputs pay for the low parts of K. Measured (D = 128 unless stated, bf16 caches,
+// us, before -> now): 32 queries x 4096 keys x 32 heads 111 -> 21, 1 x 8192 x 32
+// 209 -> 29, 128 x 4096 x 32 111 -> 33, 256 x 256 x 32 19 -> 11, D = 64 2048 x 2048 x 8
+// 48 -> 33, 500 x 500 x 16 of fp32 inputs 25.5 -> 11.
+int attn_parts(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, int sdt) {
+  const int forced = g_force_parts.load(std::memory_order_relaxed);
+  if (forced < 0) return 0;
+  const int64_t units = ceil_div(Sq, 32) * H * B;
+  const int64_t halves = 2 * ceil_div(Skv, BN) + 6;  // at most (four precisions)
+  const int64_t most = std::min<int64_t>(ceil_div(halves, ShortCfg<64>::NW), 64);
+  if (units * most >= ((int64_t)1 << 24)) return 0;
+  if (forced > 0) return (int)std::min<int64_t>(forced, most);
+  const double lo = sdt == SI_DT_F32 ? 1.45 : 1.0;
+  double best = 0.0;
+  int parts = 0;
+  for (int64_t n = 1; n <= most; ++n) {
+    const double bytes = 8.0 * 32.0 * (double)D * (double)(units * n);
+    const double t = (double)ceil_div(units * n, 256) *
+                         (6.0 + (D == 128 ? 2.15 : 1.3) * lo * (double)ceil_div(halves, ShortCfg<64>::NW * n)) +
+                     (n > 1 ? 3.5 + bytes / 3.0e6 : 0.0);
+    if (parts == 0 || t < best) { best = t; parts = (int)n; }
+  }
+  const int64_t blocks = ceil_div(Sq, 256) * H * B;
+  const double tile = (blocks > 128 ? 1.25 : 1.0) * (D == 128 ? 1.6 : 1.1) * lo;
+  const double full = (double)ceil_div(blocks, 256) * (9.0 + tile * 0.5 * (double)halves);
+  return best < full ? parts : 0;
+}
+
+// Workspace of the parts: the partial rows, then their (m, l).
+size_t parts_bytes(int parts, int64_t B, int64_t H, int64_t Sq, int64_t D) {
+  if (parts <= 1) return 0;
+  return (size_t)(ceil_div(Sq, 32) * H * B) * (size_t)parts * 32 * (size_t)(D + 2) * sizeof(float);
+}
+
+template <int D>
+void launch_short(int qdt, int sdt, int parts, hipStream_t st, const uint16_t* q, int64_t B, int64_t H,
+                  int64_t Sq, int64_t cap, const int32_t* counts, const int32_t* lists,
+                  const Buckets& bk, int64_t g, float scale_log2, void* out, int odt,
+                  const OutStrides& os, bool o32, void* ws) {
+  const int nq = (int)ceil_div(Sq, 32);
+  const int64_t units = (int64_t)nq * H * B;
+  const dim3 grid((unsigned)(units * parts));
+  float* part = reinterpret_cast<float*>(ws);
+  float* ml = part + (parts > 1 ? units * parts * 32 * D : 0);
+#define SI_SHORT(SDT_)                                                                           \
+  if (o32)                                                                                       \
+    attn_packed_short<D, SDT_, true><<<grid, 512, 0, st>>>(q, qdt, B, H, Sq, cap, counts, lists, \
+        bk, g, scale_log2, out, odt, os, nq, parts, part, ml);                              \
+  else                                                                                           \
+    attn_packed_short<D, SDT_, false><<<grid, 512, 0, st>>>(q, qdt, B, H, Sq, cap, counts, lists,\
+        bk, g, scale_log2, out, odt, os, nq, parts, part, ml)
+  switch (sdt) {
+    case SI_DT_F32: SI_SHORT(SI_DT_F32); break;
+    case SI_DT_F16: SI_SHORT(SI_DT_F16); break;
+    default: SI_SHORT(SI_DT_BF16);
+  }
+#undef SI_SHORT
+  if (parts > 1)
+    attn_combine<D><<<(unsigned)(units * 8), 64, 0, st>>>(part, ml, parts, nq, H, Sq, counts, out, odt, os);
+}
+
 }  // namespace
 }  // namespace si
 
 using namespace si;
+
+extern "C" void si_tune_attn_parts(int parts) {
+  g_force_parts.store(parts < 0 ? -1 : parts, std::memory_order_relaxed);
+}
+
+extern "C" size_t si_attn_parts_bytes(int64_t B, int64_t H, int64_t S_q, int64_t D, int64_t S_kv,
+                                      int scale_dtype) {
+  if (B <= 0 || H <= 0 || S_q <= 0 || S_kv <= 0 || (D != 64 && D != 128)) return 0;
+  return parts_bytes(attn_parts(B, H, S_q, D, S_kv, scale_dtype), B, H, S_q, D);
+}
 
 extern "C" void si_tune_attn_offset64(int on) {
   g_force_offset64.store(on != 0 ? 1 : 0, std::memory_order_relaxed);
@@ -1064,7 +1571,7 @@ int run_attn(const void* q, int q_dtype, int64_t B, int64_t H, int64_t S_q, int6
              const int8_t* code, const int32_t* slot, const void* const* buckets, int scale_dtype,
              int64_t S_kv, int64_t group, float sm_scale, void* out, int out_dtype,
              const OutStrides& os, void* workspace, size_t workspace_bytes, bool build_lists,
-             hipStream_t st) {
+             bool split, void* parts_ws, size_t parts_ws_bytes, hipStream_t st) {
   SI_CHECK_ARG(q_dtype == SI_DT_BF16 || q_dtype == SI_DT_F16,
                "si_attn_packed_fwd: q dtype must be bf16 or fp16 (got %d)", q_dtype);
   SI_CHECK_ARG(dtype_ok(scale_dtype), "si_attn_packed_fwd: unsupported scale dtype %d",
@@ -1104,6 +1611,26 @@ int run_attn(const void* q, int q_dtype, int64_t B, int64_t H, int64_t S_q, int6
   const dim3 grid((unsigned)ceil_div(S_q, bmq), (unsigned)H, (unsigned)B);
   const float scale_log2 = sm_scale * 1.4426950408889634f;
   const uint16_t* qp = reinterpret_cast<const uint16_t*>(q);
+  // The wave-per-half-tile kernel where attn_parts expects it to be faster. It
+  // reads 16 bytes of a row per lane and one int4 scale per 8 dims: buckets at
+  // other alignments (handed over by a caller) and groups that are no multiple of
+  // 8 stay with attn_packed_fwd, as do calls without a workspace for the parts
+  // and those that ask for one kernel at every size (split false).
+  int parts = split && group % 8 == 0 ? attn_parts(B, H, S_q, D, S_kv, scale_dtype) : 0;
+  for (int j = 0; j < 16; ++j)
+    if (j % 4 < 2 && (reinterpret_cast<uintptr_t>(bk.p[j]) & 15) != 0) parts = 0;
+  if (parts > 1 && (parts_ws == nullptr || (reinterpret_cast<uintptr_t>(parts_ws) & 15) != 0 ||
+                    parts_ws_bytes < parts_bytes(parts, B, H, S_q, D)))
+    parts = 0;
+  if (parts > 0) {
+#define SI_SHORT_ARGS \
+  q_dtype, scale_dtype, parts, st, qp, B, H, S_q, cap, counts, lists, bk, group, scale_log2, out, out_dtype, os, \
+  offsets32(S_kv * H, B, D), parts_ws
+    if (D == 128) launch_short<128>(SI_SHORT_ARGS);
+    else launch_short<64>(SI_SHORT_ARGS);
+#undef SI_SHORT_ARGS
+    return check_launch("si_attn_packed_fwd");
+  }
   if (D == 128) {
     if (q_dtype == SI_DT_BF16)
       launch_attn<128, SI_DT_BF16>(scale_dtype, grid, st, qp, B, H, S_q, cap, counts, lists, bk,
@@ -1132,7 +1659,7 @@ extern "C" int si_attn_packed_fwd(const void* q, int q_dtype, int64_t B, int64_t
   const OutStrides os{H * S_q * D, S_q * D, D};
   return run_attn(q, q_dtype, B, H, S_q, D, code, slot, buckets, scale_dtype, S_kv, group,
                   sm_scale, out, out_dtype, os, workspace, workspace_bytes, true,
-                  as_stream(stream));
+                  true, nullptr, 0, as_stream(stream));
 }
 
 extern "C" int si_attn_packed_fwd_tokens(const void* q, int q_dtype, int64_t B, int64_t H,
@@ -1146,7 +1673,7 @@ extern "C" int si_attn_packed_fwd_tokens(const void* q, int q_dtype, int64_t B, 
   const OutStrides os{S_q * H * D, D, H * D};
   return run_attn(q, q_dtype, B, H, S_q, D, code, slot, buckets, scale_dtype, S_kv, group,
                   sm_scale, out, out_dtype, os, workspace, workspace_bytes, true,
-                  as_stream(stream));
+                  true, nullptr, 0, as_stream(stream));
 }
 
 extern "C" int si_attn_build_lists(const int8_t* code, const int32_t* slot, int64_t H,
@@ -1179,5 +1706,20 @@ extern "C" int si_attn_packed_fwd_built(const void* q, int q_dtype, int64_t B, i
                                     : OutStrides{H * S_q * D, S_q * D, D};
   return run_attn(q, q_dtype, B, H, S_q, D, nullptr, nullptr, buckets, scale_dtype, S_kv, group,
                   sm_scale, out, out_dtype, os, const_cast<void*>(lists), lists_bytes, false,
-                  as_stream(stream));
+                  true, nullptr, 0, as_stream(stream));
+}
+
+extern "C" int si_attn_packed_fwd_parts(const void* q, int q_dtype, int64_t B, int64_t H,
+                                        int64_t S_q, int64_t D, const void* lists,
+                                        size_t lists_bytes, const void* const* buckets,
+                                        int scale_dtype, int64_t S_kv, int64_t group,
+                                        float sm_scale, void* out, int out_dtype, int token_major,
+                                        int split, void* workspace, size_t workspace_bytes,
+                                        si_stream_t stream) {
+  clear_error();
+  const OutStrides os = token_major ? OutStrides{S_q * H * D, D, H * D}
+                                    : OutStrides{H * S_q * D, S_q * D, D};
+  return run_attn(q, q_dtype, B, H, S_q, D, nullptr, nullptr, buckets, scale_dtype, S_kv, group,
+                  sm_scale, out, out_dtype, os, const_cast<void*>(lists), lists_bytes, false,
+                  split != 0, workspace, workspace_bytes, as_stream(stream));
 }

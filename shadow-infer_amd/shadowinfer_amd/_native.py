@@ -44,6 +44,7 @@ _SIGNATURES = {
     "si_check_bf16_convert": (_i32, [_vp, _vp]),
     "si_tune_gemm_plan": (None, [_i32, _i32]),
     "si_tune_attn_offset64": (None, [_i32]),
+    "si_tune_attn_parts": (None, [_i32]),
     "si_plan_workspace_bytes": (_sz, [_i64]),
     "si_plan_scan": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),
     "si_plan_scatter": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp, _vp]),
@@ -83,6 +84,10 @@ _SIGNATURES = {
     "si_attn_build_lists": (_i32, [_vp, _vp, _i64, _i64, _vp, _sz, _vp]),
     "si_attn_packed_fwd_built": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _vp, _sz, _vp, _i32,
                                         _i64, _i64, ctypes.c_float, _vp, _i32, _i32, _vp]),
+    "si_attn_parts_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i32]),
+    "si_attn_packed_fwd_parts": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _vp, _sz, _vp, _i32,
+                                        _i64, _i64, ctypes.c_float, _vp, _i32, _i32, _i32, _vp,
+                                        _sz, _vp]),
     "si_quant_rows_i8": (_i32, [_vp, _i32, _i64, _i64, _vp, _vp, _vp]),
     "si_quant_rows_i4": (_i32, [_vp, _i32, _i64, _i64, _i64, _vp, _vp, _vp]),
     "si_int4_pack_rows": (_i32, [_vp, _i64, _i64, _vp, _vp]),

@@ -169,7 +169,11 @@ class PackedDiffusionLlama:
             q, k, v = row_ops.rope_split(qkv, cos, sin, B, S, H, D)
             cache = PackedKVCache.pack(k, v, None, group_size=c.int4_group_size,
                                        plan=plan)["packed_kv"]
-        attn = packed_attention(q, cache, out_dtype=self.dtype, token_major=True)
+        # one attention kernel at every length: a row rounded otherwise flips int4
+        # codes of the next layer's cache, which shows in the logits (4% after two
+        # layers), so splitting the keys would make a trajectory depend on the shape
+        attn = packed_attention(q, cache, out_dtype=self.dtype, token_major=True,
+                                split_keys=False)
         o = F.linear(attn.view(T, Hd), L.w_o)
         y2, qx, sx, x1 = row_ops.rmsnorm(x, L.ln2, c.rms_norm_eps, want_y=trace is not None,
                                          want_q=True, residual=o)

@@ -21,13 +21,18 @@ from .packed_kv_cache import PackedKVCache
 
 def packed_attention(q: torch.Tensor, cache: PackedKVCache, sm_scale: Optional[float] = None,
                      out_dtype: torch.dtype = torch.float32,
-                     token_major: bool = False) -> torch.Tensor:
+                     token_major: bool = False, split_keys: bool = True) -> torch.Tensor:
     """``q`` ``[B, H, S_q, D]`` (bf16 or fp16) against the cache's K/V
     ``[B, H, S_kv, D]``; returns ``[B, H, S_q, D]`` in ``out_dtype`` (fp32 by
     default, the dtype of attention over the fp32 tensors unpack() returns).
     ``token_major=True`` returns ``[B, S_q, H, D]`` instead, written directly
     by the kernel: the ``attn.transpose(1, 2)`` layout an output projection
-    reads (models/diffusion_llama.py:390-391)."""
+    reads (models/diffusion_llama.py:390-391).
+
+    Calls with few queries or heads have their keys split over workgroups, and
+    then round P at other running maxima (the error against float64 is the
+    same). ``split_keys=False`` keeps one kernel, and so the same bits for a
+    query row, at every ``S_q`` and ``H``."""
     if q.dim() != 4:
         raise ValueError(f"q must be [batch, heads, seq, dim], got {tuple(q.shape)}")
     B, H, Sq, D = q.shape
@@ -47,8 +52,13 @@ def packed_attention(q: torch.Tensor, cache: PackedKVCache, sm_scale: Optional[f
     shape = (B, Sq, H, D) if token_major else (B, H, Sq, D)
     out = torch.empty(shape, dtype=out_dtype, device=qc.device)
     lists = cache.attention_lists()
-    _native.call("si_attn_packed_fwd_built", qc.data_ptr(), _native.dtype_code(q.dtype), B, H,
+    # partial results of calls whose keys are split over workgroups
+    ws_bytes = (_native.size_query("si_attn_parts_bytes", B, H, Sq, D, cache.seq_len, sdt)
+                if split_keys else 0)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=qc.device) if ws_bytes else None
+    _native.call("si_attn_packed_fwd_parts", qc.data_ptr(), _native.dtype_code(q.dtype), B, H,
                  Sq, D, lists.data_ptr(), lists.numel(), table, sdt, cache.seq_len, group,
                  float(sm_scale), out.data_ptr(), _native.dtype_code(out_dtype),
-                 1 if token_major else 0, _native.stream(q.device))
+                 1 if token_major else 0, 1 if split_keys else 0, _native.ptr(ws), ws_bytes,
+                 _native.stream(q.device))
     return out

@@ -219,3 +219,56 @@ def test_attention_extreme_scales(dev):
     ref = O.attention(q.float().numpy().reshape(B * H, S, D), rk.reshape(B * H, S, D),
                       rv.reshape(B * H, S, D)).reshape(B, H, S, D)
     assert _rel_l2(out.float().cpu(), ref) <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [1, 2, 3, 64])
+@pytest.mark.parametrize("B,H,Sq,S,D,dtype,g,probs,evicted", [
+    (1, 2, 1, 1, 128, torch.bfloat16, 16, (1, 1, 1, 1), 0.0),      # one key, one query
+    (2, 3, 33, 31, 64, torch.float32, 8, (1, 1, 1, 1), 0.2),       # half a tile, ragged queries
+    (1, 2, 32, 65, 128, torch.float32, 16, (1, 1, 1, 1), 0.1),     # a key past the first tile
+    (2, 2, 31, 500, 128, torch.float16, 32, (0, 1, 2, 1), 0.1),    # groups wider than 8 dims
+    (1, 3, 70, 700, 64, torch.bfloat16, 64, (1, 1, 2, 1), 0.05),
+    (1, 1, 5, 1500, 128, torch.bfloat16, 8, (0, 0, 1, 0), 0.0),    # one precision only
+    (1, 2, 9, 96, 64, torch.float16, 16, (1, 1, 1, 1), 1.0),       # every key evicted
+])
+def test_attention_split_keys_match_oracle(dev, parts, B, H, Sq, S, D, dtype, g, probs, evicted):
+    """The wave-per-half-tile kernel (few query blocks) at the edges of its half
+    tiles and parts, forced on by si_tune_attn_parts, in both layouts and with
+    both row offset widths (equal bits).
+
+    Bound: it multiplies the same fp16 operands as the 256-query kernel (Q, K and
+    V round alike) and differs in P's rounding alone, at another running max:
+    2^-11 relative in each kernel. So it may be 2^-11 further from the oracle
+    than that kernel is, and the two differ by at most 2^-10."""
+    k, v = kv_inputs(B, H, S, D, dtype, seed=S + D, outlier_frac=0.01)
+    codes = mixed_codes(S, H, seed=S + parts, probs=probs, sink=0 if evicted == 1.0 else 1,
+                        evicted=evicted)
+    if evicted == 1.0:
+        codes[:] = 4
+    cache = _pack(k, v, codes, dev, group_size=g)
+    q = torch.randn(B, H, Sq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
+    rk, rv = O.kv_unpack(oracle_pack(k, v, codes, group_size=g))
+    want = O.attention(q.float().numpy().reshape(B * H, Sq, D), rk.reshape(B * H, S, D),
+                       rv.reshape(B * H, S, D)).reshape(B, H, Sq, D).astype(np.float64)
+    lib = _native.load()
+    try:
+        lib.si_tune_attn_parts(-1)
+        main = packed_attention(q.to(dev), cache).cpu().double().numpy()
+        lib.si_tune_attn_parts(parts)
+        got = packed_attention(q.to(dev), cache)
+        token_major = packed_attention(q.to(dev), cache, token_major=True)
+        lib.si_tune_attn_offset64(1)
+        wide = packed_attention(q.to(dev), cache)
+    finally:
+        lib.si_tune_attn_offset64(0)
+        lib.si_tune_attn_parts(0)
+    x = got.cpu().double().numpy()
+    if evicted == 1.0:
+        assert np.array_equal(x, np.zeros_like(x))
+    else:
+        size = np.linalg.norm(want)
+        assert np.linalg.norm(x - want) <= np.linalg.norm(main - want) + 2.0 ** -11 * size
+        assert np.linalg.norm(x - main) <= 2.0 ** -10 * size
+    assert torch.equal(token_major.transpose(1, 2), got)
+    assert torch.equal(wide, got)
