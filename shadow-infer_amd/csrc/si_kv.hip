@@ -211,14 +211,17 @@ __device__ __forceinline__ void copy_words(const float* f, uint32_t* w) {
 template <int DT, int LPR, bool WC>
 __device__ __forceinline__ void pack_row(const float* xk, const float* xv, int c, int s, int b,
                                          int B, int lane, int lpg, const Buckets& bk,
-                                         uint32_t* ck, uint32_t* cv) {
+                                         uint32_t* ck, uint32_t* cv, int nl = LPR) {
   constexpr int EPL = Chunk<DT>::EPL;
-  constexpr int D = EPL * LPR;
+  const int D = EPL * nl;
+  const bool on = lane < nl;  // lanes past the row hold zeros and store nothing
   const int64_t orow = (int64_t)s * B + b;
   const int64_t oel = orow * D + lane * EPL;
   if (c == SI_PREC_FP32) {
-    store_f32<EPL>(reinterpret_cast<float*>(bk.p[0]) + oel, xk);
-    store_f32<EPL>(reinterpret_cast<float*>(bk.p[1]) + oel, xv);
+    if (on) {
+      store_f32<EPL>(reinterpret_cast<float*>(bk.p[0]) + oel, xk);
+      store_f32<EPL>(reinterpret_cast<float*>(bk.p[1]) + oel, xv);
+    }
     if constexpr (WC) {
       copy_words<DT>(xk, ck);
       copy_words<DT>(xv, cv);
@@ -226,8 +229,10 @@ __device__ __forceinline__ void pack_row(const float* xk, const float* xv, int c
     return;
   }
   if (c == SI_PREC_FP16) {
-    store_f16<EPL>(reinterpret_cast<uint16_t*>(bk.p[4]) + oel, xk);
-    store_f16<EPL>(reinterpret_cast<uint16_t*>(bk.p[5]) + oel, xv);
+    if (on) {
+      store_f16<EPL>(reinterpret_cast<uint16_t*>(bk.p[4]) + oel, xk);
+      store_f16<EPL>(reinterpret_cast<uint16_t*>(bk.p[5]) + oel, xv);
+    }
     if constexpr (WC) {
       float fk[EPL], fv[EPL];
 #pragma unroll
@@ -284,6 +289,7 @@ __device__ __forceinline__ void pack_row(const float* xk, const float* xv, int c
     copy_words<DT>(fk2, ck);
     copy_words<DT>(fv2, cv);
   }
+  if (!on) return;
   if (i8) {
     store_i8<EPL>(reinterpret_cast<int8_t*>(bk.p[8]) + oel, qk);
     store_i8<EPL>(reinterpret_cast<int8_t*>(bk.p[9]) + oel, qv);
@@ -297,7 +303,7 @@ __device__ __forceinline__ void pack_row(const float* xk, const float* xv, int c
     store_i4<EPL>(reinterpret_cast<uint8_t*>(bk.p[12]) + boff, qk);
     store_i4<EPL>(reinterpret_cast<uint8_t*>(bk.p[13]) + boff, qv);
     if ((lane & (lpg - 1)) == 0) {
-      const int64_t si = orow * (LPR / lpg) + lane / lpg;
+      const int64_t si = orow * (nl < lpg ? 1 : nl / lpg) + lane / lpg;
       store_scalar<DT>(bk.p[14], si, sk);
       store_scalar<DT>(bk.p[15], si, sv);
     }
@@ -441,12 +447,14 @@ template <int LPR, bool WC, bool DEV = false>
 __device__ __forceinline__ void pack_row_bf16(const uint32_t wk[4], const uint32_t wv[4], int c,
                                               int s, int b, int B, int lane, int lpg,
                                               const Buckets& bk, uint32_t* ck, uint32_t* cv,
-                                              int64_t row0 = 0) {
-  constexpr int D = 8 * LPR;
+                                              int64_t row0 = 0, int nl = LPR) {
+  const int D = 8 * nl;
+  const bool on = lane < nl;  // lanes past the row hold zeros and store nothing
   const int64_t orow = (int64_t)s * B + b;
   const int64_t oel = orow * D + lane * 8;
   const uint32_t rel = (uint32_t)((orow - row0) * D + lane * 8);  // element offset from row0
   if (c == SI_PREC_FP16 || c == SI_PREC_FP32) {
+    if (!on) return;
     float xk[8], xv[8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -522,6 +530,7 @@ __device__ __forceinline__ void pack_row_bf16(const uint32_t wk[4], const uint32
       cv[i] = codes_bf16x2(qv[2 * i], qv[2 * i + 1]);
     }
   }
+  if (!on) return;
   if (i8) {
     const u32x2_t k8{bytes4(qk[0], qk[1], qk[2], qk[3]), bytes4(qk[4], qk[5], qk[6], qk[7])};
     const u32x2_t v8{bytes4(qv[0], qv[1], qv[2], qv[3]), bytes4(qv[4], qv[5], qv[6], qv[7])};
@@ -557,7 +566,7 @@ __device__ __forceinline__ void pack_row_bf16(const uint32_t wk[4], const uint32
       st_row(reinterpret_cast<uint8_t*>(bk.p[13]) + boff, v4);
     }
     if ((lane & (lpg - 1)) == 0) {
-      const int64_t si = orow * (LPR / lpg) + lane / lpg;
+      const int64_t si = orow * (nl < lpg ? 1 : nl / lpg) + lane / lpg;
       reinterpret_cast<uint16_t*>(bk.p[14])[si] = (uint16_t)(__float_as_uint(sk) >> 16);
       reinterpret_cast<uint16_t*>(bk.p[15])[si] = (uint16_t)(__float_as_uint(sv) >> 16);
     }
@@ -722,8 +731,8 @@ __device__ __forceinline__ void rope_chunk(float* x, int64_t t, int lane, const 
 // Element offsets of this lane's K and V chunks of row (bb, flat = h*S + t):
 // dense [B, H, S, D] tensors, or the q|k|v projection rows with ROPE (t is
 // then returned for the cos/sin tables).
-template <bool ROPE, int D, int EPL>
-__device__ __forceinline__ void row_offsets(int64_t bb, int64_t flat, int64_t HS, int lane,
+template <bool ROPE, int EPL>
+__device__ __forceinline__ void row_offsets(int D, int64_t bb, int64_t flat, int64_t HS, int lane,
                                             const RopeSrc& rs, int64_t& koff, int64_t& voff,
                                             int64_t& t) {
   if constexpr (ROPE) {
@@ -737,14 +746,14 @@ __device__ __forceinline__ void row_offsets(int64_t bb, int64_t flat, int64_t HS
   }
 }
 
-template <int DT, int LPR, int U, int P, int NT, bool ROPE>
+template <int DT, int LPR, int U, int P, int NT, bool ROPE, bool PAD>
 __device__ __forceinline__ void pack_bucket_rows(const void* __restrict__ kin,
                                                  const void* __restrict__ vin,
                                                  const UnpackLists& L, int64_t lb, int B,
                                                  int64_t HS, int lpg, const Buckets& bk,
-                                                 const RopeSrc& rs) {
+                                                 const RopeSrc& rs, int nl) {
   constexpr int EPL = Chunk<DT>::EPL;
-  constexpr int D = EPL * LPR;
+  const int D = EPL * nl;
   constexpr int RPP = NT / LPR;
   const int lane = threadIdx.x % LPR;
   const int64_t rows = L.n[P] * B;
@@ -762,15 +771,16 @@ __device__ __forceinline__ void pack_bucket_rows(const void* __restrict__ kin,
       const int64_t r = r0 + u * RPP;
       sl[u] = -1;
       tk[u] = 0;
-      if constexpr (ROPE) {  // rows past the end still take part in the lane exchange
+      if constexpr (ROPE || PAD) {  // such lanes still take part in the lane exchanges
 #pragma unroll
         for (int i = 0; i < 4; ++i) wk[u][i] = wv[u][i] = 0u;
       }
       if (r < rows) {
         sl[u] = r / B;
         bb[u] = r - sl[u] * B;
+        if (PAD && lane >= nl) continue;
         int64_t ko, vo;
-        row_offsets<ROPE, D, EPL>(bb[u], L.flat[P][sl[u]], HS, lane, rs, ko, vo, tk[u]);
+        row_offsets<ROPE, EPL>(D, bb[u], L.flat[P][sl[u]], HS, lane, rs, ko, vo, tk[u]);
         const u32x4 a = __builtin_nontemporal_load(
             reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(kin) + ko * 2));
         const u32x4 b = __builtin_nontemporal_load(
@@ -801,7 +811,7 @@ __device__ __forceinline__ void pack_bucket_rows(const void* __restrict__ kin,
     for (int u = 0; u < U; ++u)
       if (sl[u] >= 0)
         pack_row_bf16<LPR, false, true>(wk[u], wv[u], P, (int)sl[u], (int)bb[u], B, lane, lpg, bk,
-                                        nullptr, nullptr, lb * (RPP * U));
+                                        nullptr, nullptr, lb * (RPP * U), nl);
   } else {
     float xk[U][EPL], xv[U][EPL];
     int64_t sl[U], bb[U], tk[U];
@@ -810,15 +820,16 @@ __device__ __forceinline__ void pack_bucket_rows(const void* __restrict__ kin,
       const int64_t r = r0 + u * RPP;
       sl[u] = -1;
       tk[u] = 0;
-      if constexpr (ROPE) {
+      if constexpr (ROPE || PAD) {
 #pragma unroll
         for (int e = 0; e < EPL; ++e) xk[u][e] = xv[u][e] = 0.0f;
       }
       if (r < rows) {
         sl[u] = r / B;
         bb[u] = r - sl[u] * B;
+        if (PAD && lane >= nl) continue;
         int64_t ko, vo;
-        row_offsets<ROPE, D, EPL>(bb[u], L.flat[P][sl[u]], HS, lane, rs, ko, vo, tk[u]);
+        row_offsets<ROPE, EPL>(D, bb[u], L.flat[P][sl[u]], HS, lane, rs, ko, vo, tk[u]);
         load_chunk<DT>(kin, ko, xk[u]);
         load_chunk<DT>(vin, vo, xv[u]);
       }
@@ -831,28 +842,31 @@ __device__ __forceinline__ void pack_bucket_rows(const void* __restrict__ kin,
     for (int u = 0; u < U; ++u)
       if (sl[u] >= 0)
         pack_row<DT, LPR, false>(xk[u], xv[u], P, (int)sl[u], (int)bb[u], B, lane, lpg, bk,
-                                 nullptr, nullptr);
+                                 nullptr, nullptr, nl);
   }
 }
 
-template <int DT, int LPR, int U, int NT, bool ROPE = false>
+// LPR lanes per row; with PAD only the first `active` of them hold a chunk (D is
+// EPL * active, no power of two), else active is LPR.
+template <int DT, int LPR, int U, int NT, bool ROPE = false, bool PAD = false>
 __global__ __launch_bounds__(NT) void kv_pack_lists(const void* __restrict__ kin,
                                                      const void* __restrict__ vin, UnpackLists L,
                                                      int B, int H, int S, int lpg, Buckets bk,
-                                                     RopeSrc rs = RopeSrc{}) {
+                                                     RopeSrc rs = RopeSrc{}, int active = LPR) {
+  const int nl = PAD ? active : LPR;
   const int64_t blk = blockIdx.x;
   const int64_t HS = (int64_t)H * S;
   if (blk < L.blk_end[0]) {
-    pack_bucket_rows<DT, LPR, U, SI_PREC_FP32, NT, ROPE>(kin, vin, L, blk, B, HS, lpg, bk, rs);
+    pack_bucket_rows<DT, LPR, U, SI_PREC_FP32, NT, ROPE, PAD>(kin, vin, L, blk, B, HS, lpg, bk, rs, nl);
   } else if (blk < L.blk_end[1]) {
-    pack_bucket_rows<DT, LPR, U, SI_PREC_FP16, NT, ROPE>(kin, vin, L, blk - L.blk_end[0], B, HS,
-                                                         lpg, bk, rs);
+    pack_bucket_rows<DT, LPR, U, SI_PREC_FP16, NT, ROPE, PAD>(kin, vin, L, blk - L.blk_end[0], B, HS,
+                                                         lpg, bk, rs, nl);
   } else if (blk < L.blk_end[2]) {
-    pack_bucket_rows<DT, LPR, U, SI_PREC_INT8, NT, ROPE>(kin, vin, L, blk - L.blk_end[1], B, HS,
-                                                         lpg, bk, rs);
+    pack_bucket_rows<DT, LPR, U, SI_PREC_INT8, NT, ROPE, PAD>(kin, vin, L, blk - L.blk_end[1], B, HS,
+                                                         lpg, bk, rs, nl);
   } else {
-    pack_bucket_rows<DT, LPR, U, SI_PREC_INT4, NT, ROPE>(kin, vin, L, blk - L.blk_end[2], B, HS,
-                                                         lpg, bk, rs);
+    pack_bucket_rows<DT, LPR, U, SI_PREC_INT4, NT, ROPE, PAD>(kin, vin, L, blk - L.blk_end[2], B, HS,
+                                                         lpg, bk, rs, nl);
   }
 }
 
@@ -1097,13 +1111,17 @@ __global__ __launch_bounds__(256) void kv_unpack_sorted(const int8_t* __restrict
 // Blocks past the buckets zero the rows of entries whose code is outside
 // 0..3 (evicted or absent). blk_end[p]: first block after precision p's.
 
-template <int D, int SDT, int U, int P, int NT>
+// DC: the head dim where it is a compile-time constant, else 0 (any multiple
+// of 4 up to 4 * NT, the block's last NT % (D / 4) threads idle).
+template <int DC, int SDT, int U, int P, int NT>
 __device__ __forceinline__ void unpack_bucket_rows(const UnpackLists& L, const Buckets& bk,
-                                                   int64_t lb, int B, int64_t HS, int g,
+                                                   int64_t lb, int B, int64_t HS, int Dr, int g,
                                                    float* __restrict__ ok, float* __restrict__ ov) {
-  constexpr int CPR = D / 4;
-  constexpr int RPP = NT / CPR;
+  const int D = DC ? DC : Dr;
+  const int CPR = D / 4;
+  const int RPP = NT / CPR;
   const int ch = threadIdx.x % CPR;
+  if (DC == 0 && (int)threadIdx.x >= RPP * CPR) return;
   const int64_t rows = L.n[P] * B;
   const int64_t r0 = lb * (RPP * U) + threadIdx.x / CPR;
   float4 rk[U], rv[U];
@@ -1132,30 +1150,32 @@ __device__ __forceinline__ void unpack_bucket_rows(const UnpackLists& L, const B
   }
 }
 
-template <int D, int SDT, int U, int NT>
+template <int DC, int SDT, int U, int NT>
 __global__ __launch_bounds__(NT) void kv_unpack_lists(UnpackLists L,
                                                        const int8_t* __restrict__ code,
-                                                       Buckets bk, int B, int H, int S, int g,
+                                                       Buckets bk, int B, int H, int S, int Dr, int g,
                                                        float* __restrict__ ok,
                                                        float* __restrict__ ov) {
   const int64_t blk = blockIdx.x;
   const int64_t HS = (int64_t)H * S;
   if (blk < L.blk_end[3]) {
     if (blk < L.blk_end[0]) {
-      unpack_bucket_rows<D, SDT, U, SI_PREC_FP32, NT>(L, bk, blk, B, HS, g, ok, ov);
+      unpack_bucket_rows<DC, SDT, U, SI_PREC_FP32, NT>(L, bk, blk, B, HS, Dr, g, ok, ov);
     } else if (blk < L.blk_end[1]) {
-      unpack_bucket_rows<D, SDT, U, SI_PREC_FP16, NT>(L, bk, blk - L.blk_end[0], B, HS, g, ok, ov);
+      unpack_bucket_rows<DC, SDT, U, SI_PREC_FP16, NT>(L, bk, blk - L.blk_end[0], B, HS, Dr, g, ok, ov);
     } else if (blk < L.blk_end[2]) {
-      unpack_bucket_rows<D, SDT, U, SI_PREC_INT8, NT>(L, bk, blk - L.blk_end[1], B, HS, g, ok, ov);
+      unpack_bucket_rows<DC, SDT, U, SI_PREC_INT8, NT>(L, bk, blk - L.blk_end[1], B, HS, Dr, g, ok, ov);
     } else {
-      unpack_bucket_rows<D, SDT, U, SI_PREC_INT4, NT>(L, bk, blk - L.blk_end[2], B, HS, g, ok, ov);
+      unpack_bucket_rows<DC, SDT, U, SI_PREC_INT4, NT>(L, bk, blk - L.blk_end[2], B, HS, Dr, g, ok, ov);
     }
     return;
   }
   // zero rows: entries e = t*H + h with a code outside 0..3
-  constexpr int CPR = D / 4;
-  constexpr int RPP = NT / CPR;
+  const int D = DC ? DC : Dr;
+  const int CPR = D / 4;
+  const int RPP = NT / CPR;
   const int ch = threadIdx.x % CPR;
+  if (DC == 0 && (int)threadIdx.x >= RPP * CPR) return;
   const int64_t e0 = (blk - L.blk_end[3]) * (RPP * U) + threadIdx.x / CPR;
   typedef float f32x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -1304,6 +1324,10 @@ constexpr int kListRows = SI_LIST_ROWS;
 // rows of B * D values reach 2^32 bytes.
 inline bool list_rows_wide(int64_t B, int64_t D) { return B * D * 4 * kListRows >= ((int64_t)1 << 32); }
 
+// Below this many blocks of rows a copy launch splits K and V over blocks (at 1026
+// the evict still gains 4% by it, the reuse loses 6%).
+constexpr int64_t kFewBlocks = 768;
+
 struct CopyLists {
   const int64_t* flat[4];  // destination slot order: h*S + t
   int64_t n[4];
@@ -1371,7 +1395,15 @@ __device__ __forceinline__ void copy_rows(void* dst, const void* src, int64_t ro
 // and the previous code equals the row's precision (apply_reuse_mask,
 // packed_kv_cache.py:791-852). Otherwise (compaction, :698-737): every row is
 // copied from src_slot[e] of the old buckets.
-template <bool REUSE, bool WIDE>
+//
+// FEW (a grid of blocks x 2, fewer than kFewBlocks blocks): a block copies K
+// (blockIdx.y 0) or V, with four units in flight per thread. Such a launch does
+// not fill the chip, so each block's chain of waits is its time. Back to back,
+// half reused / a quarter evicted: 96 blocks (B = 2, H = 12, S = 1003, D = 80)
+// reuse 6.8 -> 5.6 us, evict's copy 8.5 -> 6.7; 513 blocks 7.6 -> 7.3, 10.3 ->
+// 8.7. At 2049 blocks resolving the rows twice costs more: 16.3 -> 18.5, 22.0 ->
+// 23.3.
+template <bool REUSE, bool WIDE, bool FEW = false>
 __global__ __launch_bounds__(256) void kv_copy_lists(CopyLists L, Buckets dst, Buckets src,
                                                      const int8_t* __restrict__ src_code,
                                                      const int32_t* __restrict__ src_slot,
@@ -1441,14 +1473,16 @@ __global__ __launch_bounds__(256) void kv_copy_lists(CopyLists L, Buckets dst, B
     if ((int)threadIdx.x < rows) srcs[threadIdx.x] = ss;
   }
   __syncthreads();
+  constexpr int UNR = FEW ? 4 : SI_COPY_UNR;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    copy_rows<WIDE>(dst.p[4 * p + j], src.p[4 * p + j], geo.data_bytes[p], s0, n_rows, srcs, dr);
+  for (int i = 0; i < (FEW ? 1 : 2); ++i) {
+    const int j = FEW ? (int)blockIdx.y : i;
+    copy_rows<WIDE, UNR>(dst.p[4 * p + j], src.p[4 * p + j], geo.data_bytes[p], s0, n_rows, srcs, dr);
     if (geo.scale_bytes[p] > 0)
-      copy_rows<WIDE>(dst.p[4 * p + 2 + j], src.p[4 * p + 2 + j], geo.scale_bytes[p], s0, n_rows,
-                      srcs, dr);
+      copy_rows<WIDE, UNR>(dst.p[4 * p + 2 + j], src.p[4 * p + 2 + j], geo.scale_bytes[p], s0,
+                           n_rows, srcs, dr);
   }
-  if (REUSE && stats != nullptr && threadIdx.x == 0 && (cnt[0] | cnt[1])) {
+  if (REUSE && stats != nullptr && blockIdx.y == 0 && threadIdx.x == 0 && (cnt[0] | cnt[1])) {
     atomicAdd(stats, (unsigned long long)cnt[0]);
     atomicAdd(stats + 1, (unsigned long long)cnt[1]);
   }
@@ -1592,8 +1626,8 @@ __global__ __launch_bounds__(kEvictRows) void kv_evict_count(EvictLists L, int64
 // from pass 1's ballots, so the chunk counts, the bits and the old list are
 // loaded side by side and the mask is not read again. new_n[p] bounds every
 // slot written; rows are copied only for precisions whose new bucket pointer
-// is set.
-template <bool WIDE>
+// is set. FEW: K and V by blockIdx.y, as in kv_copy_lists.
+template <bool WIDE, bool FEW = false>
 __global__ __launch_bounds__(kEvictThreads) void kv_evict_lists(
     EvictLists L, const int32_t* __restrict__ chunk_count,
     const unsigned long long* __restrict__ chunk_bits, int64_t S, int64_t H, Buckets dst,
@@ -1650,21 +1684,25 @@ __global__ __launch_bounds__(kEvictThreads) void kv_evict_lists(
     const int64_t ns = prefix + (int64_t)k;
     if (ns < limit) {
       srcs[k] = s0 + threadIdx.x;
-      const uint32_t fu = (uint32_t)f, su = (uint32_t)S;  // S * H < 2^31
-      new_slot[(int64_t)(fu % su) * H + (fu / su)] = (int32_t)ns;
-      if (nl.flat[p] != nullptr) nl.flat[p][ns] = f;
+      if (!FEW || blockIdx.y == 0) {
+        const uint32_t fu = (uint32_t)f, su = (uint32_t)S;  // S * H < 2^31
+        new_slot[(int64_t)(fu % su) * H + (fu / su)] = (int32_t)ns;
+        if (nl.flat[p] != nullptr) nl.flat[p][ns] = f;
+      }
     }
   }
   __syncthreads();
   const int n_rows = (int)max<int64_t>(0, min<int64_t>((int64_t)tot, limit - prefix));
   if (n_rows == 0) return;
+  constexpr int UNR = FEW ? 4 : SI_COPY_UNR;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    copy_rows<WIDE>(dst.p[4 * p + j], src.p[4 * p + j], geo.data_bytes[p], prefix, n_rows, srcs,
-                    nullptr);
+  for (int i = 0; i < (FEW ? 1 : 2); ++i) {
+    const int j = FEW ? (int)blockIdx.y : i;
+    copy_rows<WIDE, UNR>(dst.p[4 * p + j], src.p[4 * p + j], geo.data_bytes[p], prefix, n_rows,
+                         srcs, nullptr);
     if (geo.scale_bytes[p] > 0)
-      copy_rows<WIDE>(dst.p[4 * p + 2 + j], src.p[4 * p + 2 + j], geo.scale_bytes[p], prefix,
-                      n_rows, srcs, nullptr);
+      copy_rows<WIDE, UNR>(dst.p[4 * p + 2 + j], src.p[4 * p + 2 + j], geo.scale_bytes[p], prefix,
+                           n_rows, srcs, nullptr);
   }
 }
 
@@ -2225,6 +2263,10 @@ extern "C" int si_kv_reuse_flat(const int64_t* const* cur_flat, const int64_t* c
     kv_copy_lists<true, true><<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(
         L, dst, to_buckets(prev_buckets), prev_code, prev_slot, mask, S, H, S_prev, geo,
         reinterpret_cast<unsigned long long*>(stats));
+  else if (blocks < kFewBlocks)
+    kv_copy_lists<true, false, true><<<dim3((unsigned)blocks, 2), 256, 0, as_stream(stream)>>>(
+        L, dst, to_buckets(prev_buckets), prev_code, prev_slot, mask, S, H, S_prev, geo,
+        reinterpret_cast<unsigned long long*>(stats));
   else
     kv_copy_lists<true, false><<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(
         L, dst, to_buckets(prev_buckets), prev_code, prev_slot, mask, S, H, S_prev, geo,
@@ -2353,6 +2395,10 @@ extern "C" int si_kv_evict_flat(const int64_t* const* old_flat, const int64_t* o
   const Buckets dst = to_buckets(new_buckets), src = to_buckets(old_buckets);
   if (B * D * 4 * kEvictRows >= ((int64_t)1 << 32))  // 32-bit unit indices up to here
     kv_evict_lists<true><<<(unsigned)chunks, kEvictThreads, 0, as_stream(stream)>>>(
+        L, chunk_counts, reinterpret_cast<const unsigned long long*>(chunk_bits), S, H, dst, src,
+        geo, nl, new_slot);
+  else if (chunks < kFewBlocks)
+    kv_evict_lists<false, true><<<dim3((unsigned)chunks, 2), kEvictThreads, 0, as_stream(stream)>>>(
         L, chunk_counts, reinterpret_cast<const unsigned long long*>(chunk_bits), S, H, dst, src,
         geo, nl, new_slot);
   else
@@ -2491,7 +2537,9 @@ extern "C" int si_kv_unpack_flat(const int8_t* code, const int32_t* slot,
   const bool vec = group % 4 == 0 &&
                    ((reinterpret_cast<uintptr_t>(out_k) | reinterpret_cast<uintptr_t>(out_v)) & 15) == 0;
   const bool small = B * H * S < ((int64_t)1 << 31) && B < ((int64_t)1 << 31);
-  if (!(vec && small && (D == 128 || D == 64)))  // other shapes: the token-order kernels
+  // Rows of fewer than 4 or more than 1024 values, and groups that straddle four
+  // of them, go to the token-order kernels.
+  if (!(vec && small && D % 4 == 0 && D <= 1024))
     return si_kv_unpack(code, slot, buckets, scale_dtype, B, H, S, D, group, out_k, out_v, stream);
   const Buckets bk = to_buckets(buckets);
   // Rows per thread (U) and threads per block (NT) of the bucket-order pack and
@@ -2522,15 +2570,19 @@ extern "C" int si_kv_unpack_flat(const int8_t* code, const int32_t* slot,
   const dim3 grid((unsigned)L.blk_end[4]);
   hipStream_t st = as_stream(stream);
 #define SI_UL(D_, SDT_) \
-  kv_unpack_lists<D_, SDT_, U, NT><<<grid, NT, 0, st>>>(L, code, bk, (int)B, (int)H, (int)S, (int)group, out_k, out_v)
+  kv_unpack_lists<D_, SDT_, U, NT><<<grid, NT, 0, st>>>(L, code, bk, (int)B, (int)H, (int)S, (int)D, (int)group, out_k, out_v)
   if (D == 128) {
     if (scale_dtype == SI_DT_F32) SI_UL(128, SI_DT_F32);
     else if (scale_dtype == SI_DT_F16) SI_UL(128, SI_DT_F16);
     else SI_UL(128, SI_DT_BF16);
-  } else {
+  } else if (D == 64) {
     if (scale_dtype == SI_DT_F32) SI_UL(64, SI_DT_F32);
     else if (scale_dtype == SI_DT_F16) SI_UL(64, SI_DT_F16);
     else SI_UL(64, SI_DT_BF16);
+  } else {
+    if (scale_dtype == SI_DT_F32) SI_UL(0, SI_DT_F32);
+    else if (scale_dtype == SI_DT_F16) SI_UL(0, SI_DT_F16);
+    else SI_UL(0, SI_DT_BF16);
   }
 #undef SI_UL
   return check_launch("si_kv_unpack_flat");
@@ -2563,9 +2615,19 @@ extern "C" int si_kv_pack_flat(const void* k, const void* v, int dtype, int64_t 
   const int64_t lpr = D / epl;
   const int64_t lpg = group / epl;
   const bool aligned = ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0;
+  const bool small = B * H * S < ((int64_t)1 << 31);
   const bool fast = aligned && D % epl == 0 && pow2(lpr) && lpr >= 4 && lpr <= 64 &&
-                    group % epl == 0 && pow2(lpg) && lpg <= lpr && B * H * S < ((int64_t)1 << 31);
-  if (!fast) return si_kv_pack(k, v, dtype, B, H, S, D, group, code, slot, buckets, stream);
+                    group % epl == 0 && pow2(lpg) && lpg <= lpr && small;
+  // Rows of whole 16-byte chunks whose number is no power of two (D = 80, 96):
+  // the next power of two of lanes per row, the last ones idle. An int4 group
+  // is then a power of two of chunks, or the whole row. The token-order kernel
+  // walks such an entry with one thread: B = 2, H = 12, S = 1003, D = 80 in
+  // fp16 317 us against 9.
+  const bool pad = !fast && aligned && D % epl == 0 && lpr < 64 && small &&
+                   (group == D || (group % epl == 0 && pow2(lpg) && lpg <= lpr));
+  if (!fast && !pad) return si_kv_pack(k, v, dtype, B, H, S, D, group, code, slot, buckets, stream);
+  int64_t lanes = pad ? 4 : lpr;
+  while (lanes < lpr) lanes *= 2;
 #ifndef SI_PACK_LISTS_U
 #define SI_PACK_LISTS_U 1
 #endif
@@ -2574,7 +2636,7 @@ extern "C" int si_kv_pack_flat(const void* k, const void* v, int dtype, int64_t 
 #define SI_PACK_LISTS_NT 256
 #endif
   constexpr int NT = SI_PACK_LISTS_NT;
-  const int64_t rpb = (NT / lpr) * U;
+  const int64_t rpb = (NT / lanes) * U;
   UnpackLists L;
   int64_t acc = 0;
   for (int p = 0; p < 4; ++p) {
@@ -2587,10 +2649,15 @@ extern "C" int si_kv_pack_flat(const void* k, const void* v, int dtype, int64_t 
   if (acc == 0) return SI_OK;
   SI_CHECK_ARG(acc < ((int64_t)1 << 31), "si_kv_pack_flat: too many blocks");
   const dim3 grid((unsigned)acc);
-#define SI_PL(DT_, L_) \
-  kv_pack_lists<DT_, L_, U, NT><<<grid, NT, 0, st>>>(k, v, L, (int)B, (int)H, (int)S, (int)lpg, bk)
+  const int glanes = (int)(pad && group == D ? lanes : lpg);
+#define SI_PL(DT_, L_)                                                                           \
+  if (pad)                                                                                       \
+    kv_pack_lists<DT_, L_, U, NT, false, true><<<grid, NT, 0, st>>>(                             \
+        k, v, L, (int)B, (int)H, (int)S, glanes, bk, RopeSrc{}, (int)lpr);                       \
+  else                                                                                           \
+    kv_pack_lists<DT_, L_, U, NT><<<grid, NT, 0, st>>>(k, v, L, (int)B, (int)H, (int)S, glanes, bk)
 #define SI_PL_DT(DT_)               \
-  switch (lpr) {                    \
+  switch (lanes) {                  \
     case 4: SI_PL(DT_, 4); break;   \
     case 8: SI_PL(DT_, 8); break;   \
     case 16: SI_PL(DT_, 16); break; \

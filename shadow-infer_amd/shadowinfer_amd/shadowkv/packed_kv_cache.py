@@ -339,8 +339,7 @@ class PackedKVCache:
                     f"evict mask tensor must be [S, H], got {tuple(token_head_set.shape)}")
             if not self._buckets:
                 return 0
-            mask = token_head_set.reshape(-1).to(device=self._grouping.code.device,
-                                                 dtype=torch.uint8).contiguous()
+            mask = _mask_bytes(token_head_set, self._grouping.code.device)
         else:
             if not token_head_set or not self._buckets:
                 return 0
@@ -429,7 +428,7 @@ class PackedKVCache:
             if tuple(reuse_mask.shape) not in ((self.seq_len, self.num_heads),
                                                (self.seq_len * self.num_heads,)):
                 raise ValueError(f"reuse mask tensor must be [S, H], got {tuple(reuse_mask.shape)}")
-            mask = reuse_mask.reshape(-1).to(device=dev, dtype=torch.uint8).contiguous()
+            mask = _mask_bytes(reuse_mask, dev)
         else:
             host = self._entry_mask(reuse_mask, is_dict=True)
             if host is None:
@@ -520,6 +519,13 @@ def _pack_codes_from_map(precision_map: Dict[int, Dict[int, str]], S: int, H: in
             p = name.lower()
             codes[t * H + h] = 4 if p == EVICTED else _PREC_INDEX.get(p, 1)
     return codes
+
+
+def _mask_bytes(mask: torch.Tensor, dev: torch.device) -> torch.Tensor:
+    """An ``[S, H]`` mask as flat uint8 on ``dev``; a bool tensor's bytes are
+    taken as they are (0 or 1), without a conversion pass."""
+    flat = mask.reshape(-1).to(device=dev).contiguous()
+    return flat.view(torch.uint8) if flat.dtype == torch.bool else flat.to(torch.uint8)
 
 
 def _pack_rows(q: torch.Tensor) -> torch.Tensor:

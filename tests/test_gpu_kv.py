@@ -523,3 +523,39 @@ def test_token_and_bucket_order_copies_agree(dev, dtype, shape):
         for key in ("k", "v", "scale_k", "scale_v"):
             if da.get(key) is not None:
                 assert torch.equal(da[key], fresh[name][key]), (name, key)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,H,S,D,g", [
+    (2, 3, 37, 80, 16), (1, 5, 130, 96, 16), (1, 2, 40, 8, 16), (1, 3, 33, 24, 16),
+    (2, 2, 21, 40, 8), (1, 2, 19, 104, 16), (3, 1, 17, 160, 32), (1, 2, 9, 248, 16),
+    (1, 3, 11, 12, 16), (2, 2, 13, 20, 4), (1, 1, 5, 504, 8),
+])
+def test_rows_of_any_chunk_count_bit_exact(dev, dtype, B, H, S, D, g):
+    """Head dims that are no power of two of 16-byte chunks (bucket-order pack with
+    idle lanes, bucket-order unpack at any multiple of 4), int4 groups of a
+    power of two of chunks and of the whole row, through reuse and evict:
+    every byte equal to the oracle's."""
+    k, v = kv_inputs(B, H, S, D, dtype, seed=B * 1000 + S * 10 + D)
+    codes = mixed_codes(S, H, seed=D + S, probs=(1, 1, 1, 1), sink=1, evicted=0.1)
+    cache = _pack(k, v, codes, dev, group_size=g)
+    ref = oracle_pack(k, v, codes, group_size=g)
+    assert_cache_equal(cache, ref)
+    rk, rv = O.kv_unpack(ref)
+    k_out, v_out = cache.unpack()
+    np.testing.assert_array_equal(k_out.cpu().numpy(), rk)
+    np.testing.assert_array_equal(v_out.cpu().numpy(), rv)
+    pk, pv = kv_inputs(B, H, S, D, dtype, seed=S + D)
+    prev = _pack(pk, pv, codes, dev, group_size=g)
+    reuse = np.random.default_rng(S).random((S, H)) < 0.5
+    gone = np.random.default_rng(D).random((S, H)) < 0.3
+    cache.apply_reuse_mask(prev, torch.from_numpy(reuse).to(dev))
+    cache.evict(torch.from_numpy(gone).to(dev))
+    sel = torch.from_numpy(reuse.T.copy())[None, :, :, None]
+    want = oracle_pack(torch.where(sel, pk, k), torch.where(sel, pv, v),
+                       np.where(gone, 4, codes).astype(np.int8), group_size=g)
+    assert_cache_equal(cache, want)
+    rk, rv = O.kv_unpack(want)
+    k_out, v_out = cache.unpack()
+    np.testing.assert_array_equal(k_out.cpu().numpy(), rk)
+    np.testing.assert_array_equal(v_out.cpu().numpy(), rv)
