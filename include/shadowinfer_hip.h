@@ -569,6 +569,16 @@ int si_swiglu_quant(const void* gate_up, int dtype, int64_t M, int64_t F, void* 
 int si_row_argmax_conf(const void* logits, int dtype, int64_t M, int64_t V, int64_t* tokens,
                        void* confidence, si_stream_t stream);
 
+/* The unmasking rule of schedule_round (shadowinfer/execution/
+ * block_decoding.py:149-158) over confidences [B, W] and masked (bytes, nonzero =
+ * masked): unmask = masked and confidence >= threshold; a row with masked
+ * positions and none above unmasks the first of its largest masked confidence
+ * (fallback[b] = 1). kept = the confidences of what stays masked, else 0.
+ * threshold is already rounded to dtype. */
+int si_schedule_rows(const void* confidence, int dtype, const uint8_t* masked, int64_t B,
+                     int64_t W, float threshold, uint8_t* unmask, void* kept, uint8_t* fallback,
+                     si_stream_t stream);
+
 /* Bytes of device workspace si_reuse_drift needs (independent of n). */
 size_t si_reuse_drift_workspace_bytes(int64_t n);
 

@@ -111,6 +111,7 @@ _SIGNATURES = {
     "si_rope_split": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp]),
     "si_swiglu_quant": (_i32, [_vp, _i32, _i64, _i64, _vp, _vp, _vp, _vp]),
     "si_row_argmax_conf": (_i32, [_vp, _i32, _i64, _i64, _vp, _vp, _vp]),
+    "si_schedule_rows": (_i32, [_vp, _i32, _vp, _i64, _i64, ctypes.c_float, _vp, _vp, _vp, _vp]),
     "si_reuse_drift_workspace_bytes": (_sz, [_i64]),
     "si_reuse_drift": (_i32, [_vp, _vp, _i32, _i64, _vp, _vp, _sz, _vp]),
     "si_reuse_apply": (_i32, [_vp, _vp, _vp, _i32, _i64, _vp, _vp]),

@@ -7,10 +7,10 @@ reference computes ``probs = softmax(logits)`` in the logits' dtype and takes
 two tensors without materialising the probabilities: the confidence in the
 logits' dtype, and the first index whose rounded probability equals it (for
 bf16 logits several near-equal logits often round to the same probability,
-and the first of them wins, not the largest logit). The decision rule then
-runs as the reference's own ``[B, W]`` torch ops on those tensors, so the
-threshold is compared in the logits' dtype too and fallback ties go to the
-smallest position. Nothing is read back to the host, so a denoising loop never
+and the first of them wins, not the largest logit). The decision rule is one
+more launch over those tensors (``si_schedule_rows``); the threshold is
+compared in the logits' dtype too and fallback ties go to the smallest
+position. Nothing is read back to the host, so a denoising loop never
 waits for the GPU.
 """
 
@@ -66,18 +66,17 @@ def schedule_round(logits_block: torch.Tensor, masked: torch.Tensor,
         raise ValueError(
             f"confidence_threshold must be within (0, 1], got {confidence_threshold}")
     tokens, confidences = argmax_confidence(logits_block)
-    masked = masked.to(device=logits_block.device, dtype=torch.bool)
+    dev = logits_block.device
+    mask = masked.to(device=dev, dtype=torch.bool).contiguous()
+    unmask = torch.empty_like(mask)
+    retained = torch.empty_like(confidences)
+    fallback = torch.empty(mask.shape[0], dtype=torch.bool, device=dev)
     # a tensor in the logits' dtype against a Python float: torch compares in
     # that dtype, so the threshold is rounded to it, as in the reference
-    above = masked & (confidences >= confidence_threshold)
-    needs_fallback = masked.any(dim=1) & ~above.any(dim=1)
-    # first position of the largest masked confidence (torch.argmax's tie rule)
-    best = confidences.masked_fill(~masked, float("-inf")).argmax(dim=1, keepdim=True)
-    # the reference sets fallback_unmask[b, best[b]] for rows needing it by a
-    # boolean index; a scatter of the row flag onto zeros is the same tensor
-    # without the host read of the index
-    fallback_unmask = torch.zeros_like(above).scatter_(1, best, needs_fallback.unsqueeze(1))
-    unmask = above | fallback_unmask
-    retained = confidences * (masked & ~unmask)
+    threshold = float(torch.tensor(confidence_threshold, dtype=confidences.dtype))
+    _native.call("si_schedule_rows", confidences.data_ptr(),
+                 _native.dtype_code(confidences.dtype), mask.data_ptr(), mask.shape[0],
+                 mask.shape[1], threshold, unmask.data_ptr(), retained.data_ptr(),
+                 fallback.data_ptr(), _native.stream(dev))
     return ScheduleDecision(unmask=unmask, tokens=tokens, confidences=retained,
-                            progress_fallback=needs_fallback)
+                            progress_fallback=fallback)

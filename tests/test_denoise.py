@@ -798,3 +798,51 @@ def test_rope_pack_support_rule():
     assert not row_ops.rope_pack_supported(torch.bfloat16, 96, 16)
     assert not row_ops.rope_pack_supported(torch.bfloat16, 128, 4)
     assert row_ops.rope_pack_supported(torch.bfloat16, 64, 24)  # 24 does not divide 64: one group of D
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,V", [(3, 2034), (3, 2035), (2, 8190), (5, 16379), (4, 32754), (4, 32755),
+                                 (3, 32769), (7, 13)])
+def test_argmax_conf_row_lengths(dev, dtype, M, V):
+    """Row lengths at both sides of each register-held size and rows that start
+    between 16-byte boundaries (odd V), each row with its maximum in the first or
+    last column and the neighbouring rows' columns larger: tokens and confidences
+    as torch's softmax + max on the GPU, outside the oracle's flagged rows."""
+    from shadowinfer_amd.execution import argmax_confidence
+    g = torch.Generator().manual_seed(M * V)
+    logits = torch.randn(M, V, generator=g)
+    for m in range(M):  # rising from row to row
+        logits[m, 0 if m % 2 else V - 1] = 12.0 + m
+    logits = logits.to(dtype)
+    tok, conf = argmax_confidence(logits.to(dev))
+    rt, rc, amb = R.argmax_conf(to_np(logits), DT[dtype], return_ambiguous=True)
+    np.testing.assert_array_equal(tok.cpu().numpy()[~amb], rt[~amb])
+    if dtype == torch.float32:
+        np.testing.assert_allclose(to_np(conf), rc, rtol=4 * R.SUM_REL_ERR)
+    else:
+        np.testing.assert_array_equal(to_np(conf)[~amb], rc[~amb])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W", [1, 63, 1024, 1025, 3000])
+def test_schedule_rows_nan_ties_and_signs(dev, W):
+    """The unmasking rule with NaN confidences (largest for the fallback, NaN kept
+    confidences), ties (smallest position) and nothing masked, against the
+    reference's op sequence."""
+    from shadowinfer_amd.execution import schedule_round
+    V = 24
+    g = torch.Generator().manual_seed(W)
+    lg = (torch.randn(4, W, V, generator=g) * 0.3).to(torch.bfloat16)
+    lg[1, W // 2] = float("nan")
+    lg[2] = lg[2, :1]             # every position ties
+    lg = lg.to(dev)
+    mk = torch.rand(4, W, generator=g) < 0.5
+    mk[3] = False
+    mk[1, W // 2] = True
+    mk = mk.to(dev)
+    for thr in (0.9, 0.05):
+        d = schedule_round(lg, mk, thr)
+        ru, rt, rc, rf = _reference_schedule(lg, mk, thr)
+        assert torch.equal(d.unmask, ru) and torch.equal(d.progress_fallback, rf)
+        assert torch.equal(torch.nan_to_num(d.confidences, nan=2.0), torch.nan_to_num(rc, nan=2.0))
