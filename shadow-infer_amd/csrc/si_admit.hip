@@ -9,18 +9,30 @@
 // that covers the excess over the budget (a partial downgrade for the entry
 // at the cut), then optionally evicts a second prefix. Only the cut entry
 // matters, so the device never sorts: a weighted radix select over the
-// score keys (four 8-bit digits, most significant first) finds the key of
-// the cut entry, a scan over the entries with that key (in index order, as a
-// stable sort leaves them) finds the entry itself, and one pass rewrites the
+// score keys (digits of 11, 11 and 10 bits, most significant first) finds the
+// key of the cut entry, a scan over the entries with that key (in index order, as
+// a stable sort leaves them) finds the entry itself, and one pass rewrites the
 // codes of everything ranked before it. Every step is an integer sum, so the
 // cut is exact.
+//
+// One layer's 262144 entries are 1.5 MB: the time is launches, round trips and
+// contended atomics, not bytes. So every block of a pass takes the step before
+// it by itself (picks the digit from the histogram of the last pass, the entry
+// from the chunk sums) instead of one block in a launch of its own, the first
+// digit's histogram is part of the pass before it, threads load four entries at
+// once, and at most kAdmBlocks blocks add to the same few counters: 10 launches
+// for 30. (Handing over to the last block of a pass instead took as long as the
+// 30 launches: its device-scope fences write back and drop the L2s, 20 us each.)
+// The solver with eviction at 8192 x 32: 195 -> 55 us of kernels.
 #include "si_common.h"
 
 namespace si {
 namespace {
 
-constexpr int ADM_THREADS = 256;
-constexpr int TIE_CHUNK = 2048;  // entries per block of the tie scan
+constexpr int ADM_THREADS = 1024;
+constexpr int64_t kAdmBlocks = 64;
+constexpr int TIE_CHUNK = 2 * ADM_THREADS;  // entries per block of the tie scan
+constexpr int BINS = 2048;                  // of a digit's histogram
 constexpr int MODE_DOWN = 0;     // ladder downgrade (fp32 -> fp16 -> int8 -> int4)
 constexpr int MODE_EVICT = 1;    // eviction of the remaining bytes
 
@@ -29,19 +41,20 @@ struct AdmCosts {
   long long delta[3];  // cost[c] - cost[c + 1]
 };
 
+// What a step of a selection leaves for the next pass.
+struct Sel {
+  unsigned long long R;  // weight the cut still has to cover
+  unsigned int prefix;   // key bits fixed so far; the cut key after three digits
+  int active;            // the selection runs
+  int all;               // the whole ranking is inside the cut
+};
+
 struct AdmState {
-  unsigned long long pred[3];  // total bytes after prep, downgrade, eviction
+  unsigned long long pred[2];  // total bytes after prep, downgrade
   unsigned long long ncand;    // eligible entries
-  unsigned long long evicted;  // entries newly evicted
-  unsigned long long R;        // weight the cut still has to cover
-  unsigned long long rem;      // excess left when the ranking reaches the cut entry
   long long budget;            // bytes allowed (may be negative)
-  int use_budget;              // 0: no budget, nothing is admitted
-  long long b_idx;             // flat index of the cut entry
-  unsigned int prefix;         // key bits fixed so far; the cut key after four digits
-  int active;                  // the current selection runs
-  int all;                     // the whole ranking is inside the cut
   int bad;                     // codes outside 0..4 were seen
+  Sel sel[2][3];               // by mode, after each digit
 };
 
 // Bytes an entry of code c frees when taken down the ladder to int4.
@@ -78,254 +91,366 @@ __device__ __forceinline__ T block_sum(T v, T* red) {
   return s;
 }
 
-__global__ void adm_init(AdmState* st, unsigned long long* hist, long long budget, int use_budget) {
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) hist[i] = 0;
-  if (threadIdx.x == 0) {
-    st->pred[0] = st->pred[1] = st->pred[2] = 0;
-    st->ncand = st->evicted = st->R = st->rem = 0;
-    st->budget = budget;
-    st->use_budget = use_budget;
-    st->b_idx = -1;
-    st->prefix = 0;
-    st->active = st->all = st->bad = 0;
+// Inclusive scan of one value per thread over the block's 1024 threads.
+__device__ __forceinline__ unsigned long long block_scan(unsigned long long v,
+                                                         unsigned long long* red) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  __syncthreads();
+  if (lane == 63) red[wave] = v;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) v += red[w];
+  return v;
+}
+
+// Digit d of a key (0: bits 31..21, 1: 20..10, 2: 9..0) and the key bits above it.
+__device__ __forceinline__ unsigned int digit_of(unsigned int k, int d) {
+  return d == 0 ? k >> 21 : d == 1 ? (k >> 10) & 2047u : k & 1023u;
+}
+__device__ __forceinline__ unsigned int above_digit(unsigned int k, int d) {
+  return d == 1 ? k >> 21 : k >> 10;  // d = 1 or 2
+}
+
+// Entries i .. i+3 of an array (zeros past n), in one load where p is aligned.
+struct Four {
+  unsigned int v[4];
+};
+template <typename T>
+__device__ __forceinline__ Four load4(const T* p, int64_t i, int64_t n) {
+  Four f;
+  if (i + 4 <= n && (reinterpret_cast<uintptr_t>(p + i) & (4 * sizeof(T) - 1)) == 0) {
+    if constexpr (sizeof(T) == 1) {
+      const unsigned int w = *reinterpret_cast<const unsigned int*>(p + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f.v[e] = (unsigned int)(int)(T)(w >> (8 * e));
+    } else {
+      const uint4 w = *reinterpret_cast<const uint4*>(p + i);
+      f.v[0] = w.x; f.v[1] = w.y; f.v[2] = w.z; f.v[3] = w.w;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (sizeof(T) == 1) f.v[e] = i + e < n ? (unsigned int)(int)p[i + e] : 0u;
+      else f.v[e] = i + e < n ? __builtin_bit_cast(unsigned int, p[i + e]) : 0u;
+    }
+  }
+  return f;
+}
+__device__ __forceinline__ void store4(int8_t* p, int64_t i, int64_t n, const int (&c)[4]) {
+  if (i + 4 <= n && (reinterpret_cast<uintptr_t>(p + i) & 3) == 0) {
+    *reinterpret_cast<unsigned int*>(p + i) = (c[0] & 255) | (c[1] & 255) << 8 |
+                                              (c[2] & 255) << 16 | (unsigned int)(c[3] & 255) << 24;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i + e < n) p[i + e] = (int8_t)c[e];
   }
 }
 
-// Copies the codes, sums their bytes, and computes each entry's score key and
-// eligibility (not a sink token, not protected).
+__global__ __launch_bounds__(ADM_THREADS) void adm_init(AdmState* st, unsigned long long* hist,
+                                                        long long budget, int64_t* result) {
+  for (int i = threadIdx.x; i < 6 * BINS; i += blockDim.x) hist[i] = 0;
+  if (threadIdx.x == 0) {
+    st->pred[0] = st->pred[1] = st->ncand = 0;
+    st->budget = budget;
+    st->bad = 0;
+  }
+  if (threadIdx.x < 3) result[threadIdx.x] = 0;
+}
+
+// The bin of a histogram that holds the cut: the first where the running weight
+// reaches R (which then is what the cut still covers inside it). False in every
+// thread when all bins together weigh less.
+__device__ __forceinline__ bool pick_digit(const unsigned long long* __restrict__ hist,
+                                           unsigned long long& R, unsigned int& bin,
+                                           unsigned long long* red) {
+  __shared__ unsigned long long left;
+  __shared__ int hit;
+  const int b = 2 * threadIdx.x;
+  const unsigned long long w0 = hist[b], w1 = hist[b + 1];
+  if (threadIdx.x == 0) hit = -1;
+  const unsigned long long cum = block_scan(w0 + w1, red), before = cum - w0 - w1;
+  if (before < R && cum >= R) {
+    const bool second = before + w0 < R;
+    hit = b + (second ? 1 : 0);
+    left = R - before - (second ? w0 : 0);
+  }
+  __syncthreads();
+  const bool found = hit >= 0;
+  if (found) {
+    bin = (unsigned int)hit;
+    R = left;
+  }
+  return found;
+}
+
+// The selection after its digit d: the downgrade cuts the excess of the initial
+// bytes over the budget, the eviction the excess left after the downgrade. The
+// same in every block; the first leaves it for the next pass.
+__device__ __forceinline__ Sel step_sel(AdmState* st, int mode, int d,
+                                        const unsigned long long* __restrict__ hist,
+                                        unsigned long long* red) {
+  Sel s;
+  if (d == 0) {
+    const long long p = (long long)st->pred[mode], budget = st->budget;
+    s.active = st->ncand > 0 && st->bad == 0 && p > budget;
+    s.all = 0;
+    s.prefix = 0;
+    s.R = s.active ? (unsigned long long)p - (unsigned long long)budget : 0;
+  } else {
+    s = st->sel[mode][d - 1];
+  }
+  if (s.active && !s.all) {
+    unsigned int bin = 0;
+    if (pick_digit(hist + (3 * mode + d) * BINS, s.R, bin, red))
+      s.prefix = (s.prefix << (d == 2 ? 10 : 11)) | bin;
+    else
+      s.all = 1;  // every candidate together saves less than the excess (d = 0)
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->sel[mode][d] = s;
+  return s;
+}
+
+// Adds a block's LDS histogram to the global one.
+__device__ __forceinline__ void flush_hist(const unsigned long long* lh, unsigned long long* hist) {
+  __syncthreads();
+  for (int b = threadIdx.x; b < BINS; b += ADM_THREADS)
+    if (lh[b] != 0) atomicAdd(&hist[b], lh[b]);
+}
+
+// Sums the codes' bytes, and computes each entry's score key and eligibility
+// (not a sink token, not protected) and the first digit's histogram of the
+// downgrade's weights. out: where the call ends here (no budget), a copy of the
+// codes.
 __global__ __launch_bounds__(ADM_THREADS) void adm_prep(
-    const int8_t* __restrict__ codes_in, int8_t* __restrict__ codes, int64_t n, int64_t H,
+    const int8_t* __restrict__ codes, int8_t* __restrict__ out, int64_t n, int64_t first,
     const float* __restrict__ imp, const float* __restrict__ sens,
-    const uint8_t* __restrict__ prot, int64_t sink, AdmCosts cs, unsigned int* __restrict__ key,
-    uint8_t* __restrict__ cand, AdmState* st) {
+    const uint8_t* __restrict__ prot, AdmCosts cs, unsigned int* __restrict__ key,
+    uint8_t* __restrict__ cand, unsigned long long* __restrict__ hist, AdmState* st,
+    int64_t* __restrict__ result) {
   __shared__ unsigned long long red[ADM_THREADS / 64];
+  __shared__ unsigned long long lh[BINS];
+  for (int b = threadIdx.x; b < BINS; b += ADM_THREADS) lh[b] = 0;
+  __syncthreads();
   unsigned long long bytes = 0, nc = 0;
   int bad = 0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int c = codes_in[i];
-    codes[i] = (int8_t)c;
-    if (c < 0 || c > 4) bad = 1;
-    else bytes += (unsigned long long)cs.cost[c];
-    const bool elig = i / H >= sink && !(prot != nullptr && prot[i] != 0);
-    const float s = sens != nullptr ? imp[i] * sens[i] : imp[i];
-    key[i] = score_key(s);
-    cand[i] = elig ? 1 : 0;
-    nc += elig ? 1 : 0;
+  for (int64_t i = 4 * ((int64_t)blockIdx.x * ADM_THREADS + threadIdx.x); i < n;
+       i += 4 * (int64_t)gridDim.x * ADM_THREADS) {
+    const Four c4 = load4(codes, i, n), m4 = load4(imp, i, n);
+    Four s4 = {}, p4 = {};
+    if (sens != nullptr) s4 = load4(sens, i, n);
+    if (prot != nullptr) p4 = load4(prot, i, n);
+    int c[4];
+    unsigned int k[4], el = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      c[e] = (int)c4.v[e];
+      const float m = __uint_as_float(m4.v[e]);
+      k[e] = score_key(sens != nullptr ? m * __uint_as_float(s4.v[e]) : m);
+      if (i + e >= n) continue;
+      if (c[e] < 0 || c[e] > 4) bad = 1;
+      else bytes += (unsigned long long)cs.cost[c[e]];
+      if (i + e < first || p4.v[e] != 0) continue;
+      el |= 1u << (8 * e);
+      ++nc;
+      const unsigned long long w = weight(cs, MODE_DOWN, c[e]);
+      if (w != 0) atomicAdd(&lh[digit_of(k[e], 0)], w);
+    }
+    if (out != nullptr) store4(out, i, n, c);
+    // key and cand are padded to whole groups of four
+    *reinterpret_cast<uint4*>(key + i) = make_uint4(k[0], k[1], k[2], k[3]);
+    *reinterpret_cast<unsigned int*>(cand + i) = el;
   }
+  flush_hist(lh, hist);
   bytes = block_sum(bytes, red);
   nc = block_sum(nc, red);
   const int any_bad = __syncthreads_or(bad);
   if (threadIdx.x == 0) {
     atomicAdd(&st->pred[0], bytes);
     atomicAdd(&st->ncand, nc);
-    if (any_bad) atomicOr(&st->bad, 1);
-  }
-}
-
-// Starts a selection: the downgrade cuts the excess of the initial bytes over
-// the budget, the eviction the excess left after the downgrade.
-__global__ void adm_sel_begin(AdmState* st, int mode, int allow_evict) {
-  if (threadIdx.x != 0) return;
-  const long long budget = st->budget;
-  const long long p = (long long)(mode == MODE_DOWN ? st->pred[0] : st->pred[1]);
-  int active = st->use_budget && st->ncand > 0 && st->bad == 0 && p > budget;
-  if (mode == MODE_EVICT && !allow_evict) active = 0;
-  st->active = active;
-  st->all = 0;
-  st->prefix = 0;
-  st->b_idx = -1;
-  st->rem = 0;
-  st->R = active ? (unsigned long long)p - (unsigned long long)budget : 0;
-}
-
-// Weight histogram of one 8-bit key digit over the candidates whose higher
-// digits equal the ones already fixed.
-__global__ __launch_bounds__(ADM_THREADS) void adm_hist(
-    int mode, int digit, const unsigned int* __restrict__ key, const uint8_t* __restrict__ cand,
-    const int8_t* __restrict__ codes, int64_t n, AdmCosts cs, unsigned long long* __restrict__ hist,
-    const AdmState* st) {
-  if (!st->active || st->all) return;
-  __shared__ unsigned long long lh[256];
-  for (int b = threadIdx.x; b < 256; b += blockDim.x) lh[b] = 0;
-  __syncthreads();
-  const unsigned int prefix = st->prefix;
-  const int sh = 8 * digit;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    if (!cand[i]) continue;
-    const unsigned int k = key[i];
-    if (digit < 3 && (k >> (sh + 8)) != prefix) continue;
-    const unsigned long long w = weight(cs, mode, codes[i]);
-    if (w != 0) atomicAdd(&lh[(k >> sh) & 255u], w);
-  }
-  __syncthreads();
-  for (int b = threadIdx.x; b < 256; b += blockDim.x)
-    if (lh[b] != 0) atomicAdd(&hist[b], lh[b]);
-}
-
-// Picks the digit whose bucket holds the cut (the first bucket where the
-// running weight reaches R), and clears the histogram for the next digit.
-// One block of 256 threads.
-__global__ __launch_bounds__(256) void adm_pick(int digit, unsigned long long* hist, AdmState* st) {
-  if (!st->active || st->all) return;
-  __shared__ unsigned long long cum[256];
-  const int b = threadIdx.x;
-  cum[b] = hist[b];
-  __syncthreads();
-  for (int o = 1; o < 256; o <<= 1) {
-    const unsigned long long add = b >= o ? cum[b - o] : 0;
-    __syncthreads();
-    cum[b] += add;
-    __syncthreads();
-  }
-  hist[b] = 0;
-  const unsigned long long R = st->R;
-  if (digit == 3 && cum[255] < R) {  // every candidate together saves less than the excess
-    if (b == 0) st->all = 1;
-    return;
-  }
-  const unsigned long long before = b > 0 ? cum[b - 1] : 0;
-  if (cum[b] >= R && before < R) {
-    st->prefix = (st->prefix << 8) | (unsigned int)b;
-    st->R = R - before;
-  }
-}
-
-// Per-chunk weight of the candidates whose key equals the cut key.
-__global__ __launch_bounds__(ADM_THREADS) void adm_tie_sum(
-    int mode, const unsigned int* __restrict__ key, const uint8_t* __restrict__ cand,
-    const int8_t* __restrict__ codes, int64_t n, AdmCosts cs, unsigned long long* __restrict__ blk,
-    const AdmState* st) {
-  if (!st->active || st->all) return;
-  __shared__ unsigned long long red[ADM_THREADS / 64];
-  const unsigned int tau = st->prefix;
-  const int64_t base = (int64_t)blockIdx.x * TIE_CHUNK;
-  unsigned long long s = 0;
-  for (int64_t i = base + threadIdx.x; i < min(base + TIE_CHUNK, n); i += blockDim.x)
-    if (cand[i] && key[i] == tau) s += weight(cs, mode, codes[i]);
-  s = block_sum(s, red);
-  if (threadIdx.x == 0) blk[blockIdx.x] = s;
-}
-
-// Inclusive scan of 1024 values held one per thread; returns this thread's sum.
-__device__ __forceinline__ unsigned long long scan1024(unsigned long long v, unsigned long long* sh) {
-  const int t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const unsigned long long add = t >= o ? sh[t - o] : 0;
-    __syncthreads();
-    sh[t] += add;
-    __syncthreads();
-  }
-  const unsigned long long r = sh[t];
-  __syncthreads();
-  return r;
-}
-
-// Finds the cut entry among the candidates with the cut key, in index order:
-// the chunk whose running weight reaches R, then the entry inside it.
-// One block of 1024 threads.
-__global__ __launch_bounds__(1024) void adm_tie_pick(
-    int mode, const unsigned int* __restrict__ key, const uint8_t* __restrict__ cand,
-    const int8_t* __restrict__ codes, int64_t n, AdmCosts cs, const unsigned long long* __restrict__ blk,
-    int64_t nblk, AdmState* st) {
-  if (!st->active || st->all) return;
-  __shared__ unsigned long long sh[1024];
-  __shared__ long long found;
-  __shared__ unsigned long long carry;
-  const int t = threadIdx.x;
-  const unsigned int tau = st->prefix;
-  unsigned long long R = st->R;
-  if (t == 0) { found = -1; carry = 0; }
-  __syncthreads();
-  // 1. the chunk
-  for (int64_t c0 = 0; c0 < nblk; c0 += 1024) {
-    const int64_t c = c0 + t;
-    const unsigned long long v = c < nblk ? blk[c] : 0;
-    const unsigned long long inc = scan1024(v, sh) + carry;
-    const unsigned long long exc = inc - v;
-    if (c < nblk && inc >= R && exc < R) found = c;
-    __syncthreads();
-    if (found >= 0) {
-      if (c == found) { R -= exc; carry = R; }  // weight left inside the chunk
-      break;
+    if (any_bad) {
+      atomicOr(&st->bad, 1);
+      atomicOr(reinterpret_cast<unsigned long long*>(result) + 2, 1ull);
     }
-    if (t == 1023) carry = inc;
-    __syncthreads();
-  }
-  __syncthreads();
-  if (found < 0) return;  // cannot happen: the digits guarantee enough weight
-  R = carry;
-  const int64_t base = found * TIE_CHUNK;
-  // 2. the entry: two consecutive entries per thread keep index order
-  const int64_t i0 = base + 2 * t;
-  unsigned long long w0 = 0, w1 = 0;
-  if (i0 < n && cand[i0] && key[i0] == tau) w0 = weight(cs, mode, codes[i0]);
-  if (i0 + 1 < n && cand[i0 + 1] && key[i0 + 1] == tau) w1 = weight(cs, mode, codes[i0 + 1]);
-  const unsigned long long inc = scan1024(w0 + w1, sh);
-  const unsigned long long exc = inc - w0 - w1;
-  if (exc < R && exc + w0 >= R) {
-    st->b_idx = i0;
-    st->rem = R - exc;
-  } else if (exc + w0 < R && inc >= R) {
-    st->b_idx = i0 + 1;
-    st->rem = R - exc - w0;
+    if (out != nullptr) atomicAdd(reinterpret_cast<unsigned long long*>(result), bytes);
   }
 }
 
-// Rewrites the codes of the candidates ranked before the cut (and the cut
-// entry), then sums the new total bytes.
+// Picks digit d - 1, then makes the weight histogram of digit d (1 or 2) over the
+// candidates whose higher digits equal the ones already fixed.
+__global__ __launch_bounds__(ADM_THREADS) void adm_hist(
+    int mode, int d, const unsigned int* __restrict__ key, const uint8_t* __restrict__ cand,
+    const int8_t* __restrict__ codes, int64_t n, AdmCosts cs, unsigned long long* __restrict__ hist,
+    AdmState* st) {
+  __shared__ unsigned long long red[ADM_THREADS / 64];
+  __shared__ unsigned long long lh[BINS];
+  for (int b = threadIdx.x; b < BINS; b += ADM_THREADS) lh[b] = 0;
+  const Sel s = step_sel(st, mode, d - 1, hist, red);
+  if (!s.active || s.all) return;
+  __syncthreads();
+  for (int64_t i = 4 * ((int64_t)blockIdx.x * ADM_THREADS + threadIdx.x); i < n;
+       i += 4 * (int64_t)gridDim.x * ADM_THREADS) {
+    const Four k4 = load4(key, i, n), e4 = load4(cand, i, n), c4 = load4(codes, i, n);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (above_digit(k4.v[e], d) != s.prefix || e4.v[e] == 0) continue;
+      const unsigned long long w = weight(cs, mode, (int)c4.v[e]);
+      if (w != 0) atomicAdd(&lh[digit_of(k4.v[e], d)], w);
+    }
+  }
+  flush_hist(lh, hist + (3 * mode + d) * BINS);
+}
+
+// Weight of the candidates with the cut key among entries i .. i+1.
+__device__ __forceinline__ void tied_pair(int mode, unsigned int tau, int64_t i, int64_t n,
+                                          const unsigned int* __restrict__ key,
+                                          const uint8_t* __restrict__ cand,
+                                          const int8_t* __restrict__ codes, const AdmCosts& cs,
+                                          unsigned long long& w0, unsigned long long& w1) {
+  w0 = w1 = 0;
+  const bool a = i < n, b = i + 1 < n;
+  const unsigned int k0 = a ? key[i] : 0, k1 = b ? key[i + 1] : 0;
+  const int e0 = a ? cand[i] : 0, e1 = b ? cand[i + 1] : 0;
+  const int c0 = a ? codes[i] : 0, c1 = b ? codes[i + 1] : 0;
+  if (e0 && k0 == tau) w0 = weight(cs, mode, c0);
+  if (e1 && k1 == tau) w1 = weight(cs, mode, c1);
+}
+
+// Picks the last digit, then sums per chunk the weight of the candidates whose
+// key equals the cut key.
+__global__ __launch_bounds__(ADM_THREADS) void adm_tie(
+    int mode, const unsigned int* __restrict__ key, const uint8_t* __restrict__ cand,
+    const int8_t* __restrict__ codes, int64_t n, AdmCosts cs,
+    const unsigned long long* __restrict__ hist, unsigned long long* __restrict__ blk,
+    AdmState* st) {
+  __shared__ unsigned long long red[ADM_THREADS / 64];
+  const Sel s = step_sel(st, mode, 2, hist, red);
+  if (!s.active || s.all) return;
+  unsigned long long w0, w1;
+  tied_pair(mode, s.prefix, (int64_t)blockIdx.x * TIE_CHUNK + 2 * threadIdx.x, n, key, cand, codes,
+            cs, w0, w1);
+  const unsigned long long sum = block_sum(w0 + w1, red);
+  if (threadIdx.x == 0) blk[blockIdx.x] = sum;
+}
+
+// The cut entry among the candidates with the cut key, in index order: the chunk
+// whose running weight reaches R, then the entry inside it (two consecutive
+// entries per thread); rem: the excess left when the ranking reaches it.
+__device__ __forceinline__ void cut_entry(int mode, const Sel& s,
+                                          const unsigned int* __restrict__ key,
+                                          const uint8_t* __restrict__ cand,
+                                          const int8_t* __restrict__ codes, int64_t n,
+                                          const AdmCosts& cs,
+                                          const unsigned long long* __restrict__ blk, int64_t nblk,
+                                          unsigned long long* red, long long& b_idx,
+                                          long long& rem) {
+  __shared__ long long found, at;
+  __shared__ unsigned long long left, so_far, excess;
+  const int t = threadIdx.x;
+  if (t == 0) found = at = -1;
+  unsigned long long carry = 0;
+  for (int64_t c0 = 0; c0 < nblk; c0 += ADM_THREADS) {
+    const unsigned long long v = c0 + t < nblk ? blk[c0 + t] : 0;
+    const unsigned long long inc = block_scan(v, red) + carry;
+    if (inc >= s.R && inc - v < s.R) {
+      found = c0 + t;
+      left = s.R - (inc - v);  // weight left inside the chunk
+    }
+    if (t == ADM_THREADS - 1) so_far = inc;
+    __syncthreads();
+    if (found >= 0) break;
+    carry = so_far;
+    __syncthreads();
+  }
+  const long long chunk = found;
+  if (chunk >= 0) {  // always: the digits guarantee enough weight
+    const unsigned long long r = left;
+    const int64_t i0 = chunk * TIE_CHUNK + 2 * t;
+    unsigned long long w0, w1;
+    tied_pair(mode, s.prefix, i0, n, key, cand, codes, cs, w0, w1);
+    const unsigned long long inc = block_scan(w0 + w1, red), exc = inc - w0 - w1;
+    if (exc < r && exc + w0 >= r) {
+      at = i0;
+      excess = r - exc;
+    } else if (exc + w0 < r && inc >= r) {
+      at = i0 + 1;
+      excess = r - exc - w0;
+    }
+  }
+  __syncthreads();
+  b_idx = at;
+  rem = at >= 0 ? (long long)excess : 0;
+}
+
+// Finds the cut entry, rewrites the codes of the candidates ranked before it
+// (and its own) from `codes` to `out`, and sums the new total bytes. The
+// downgrade before an eviction (result null) also makes the first digit's
+// histogram of the eviction's weights.
 __global__ __launch_bounds__(ADM_THREADS) void adm_apply(
     int mode, const unsigned int* __restrict__ key, const uint8_t* __restrict__ cand,
-    int8_t* __restrict__ codes, int64_t n, AdmCosts cs, AdmState* st, int slot) {
+    const int8_t* __restrict__ codes, int8_t* __restrict__ out, int64_t n, AdmCosts cs,
+    unsigned long long* __restrict__ hist, const unsigned long long* __restrict__ blk, int64_t nblk,
+    AdmState* st, int64_t* __restrict__ result) {
   __shared__ unsigned long long red[ADM_THREADS / 64];
-  const int active = st->active;
-  const int all = st->all;
-  const unsigned int tau = st->prefix;
-  const long long b_idx = st->b_idx;
-  const long long rem = (long long)st->rem;
+  __shared__ unsigned long long lh[BINS];
+  const bool next = result == nullptr;
+  if (next)
+    for (int b = threadIdx.x; b < BINS; b += ADM_THREADS) lh[b] = 0;
+  const Sel s = st->sel[mode][2];
+  long long b_idx = -1, rem = 0;
+  if (s.active && !s.all) cut_entry(mode, s, key, cand, codes, n, cs, blk, nblk, red, b_idx, rem);
+  const int all = s.all;
+  const unsigned int tau = s.prefix;
+  __syncthreads();
   unsigned long long bytes = 0, ev = 0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    int c = codes[i];
-    if (active && cand[i]) {
-      const unsigned int k = key[i];
-      const bool before = all || k < tau || (k == tau && i < b_idx);
-      const bool at = !all && i == b_idx;
-      const int c0 = c;
-      if (mode == MODE_DOWN) {
-        if (before) {
-          if (c != 4) c = 3;
-        } else if (at && c != 4) {
-          const long long s1 = c < 3 ? cs.delta[c] : 0;
-          const int n1 = c < 3 ? c + 1 : c;
-          const long long s2 = n1 < 3 ? cs.delta[n1] : 0;
-          const int n2 = n1 < 3 ? n1 + 1 : n1;
-          c = rem <= s1 ? n1 : rem <= s1 + s2 ? n2 : 3;
+  for (int64_t i = 4 * ((int64_t)blockIdx.x * ADM_THREADS + threadIdx.x); i < n;
+       i += 4 * (int64_t)gridDim.x * ADM_THREADS) {
+    const Four k4 = load4(key, i, n), e4 = load4(cand, i, n), c4 = load4(codes, i, n);
+    int o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      int c = (int)c4.v[e];
+      const unsigned int k = k4.v[e];
+      const bool elig = e4.v[e] != 0;
+      if (s.active && elig) {
+        const bool before = all || k < tau || (k == tau && i + e < b_idx);
+        const bool at = !all && i + e == b_idx;
+        if (mode == MODE_DOWN) {
+          if (before) {
+            if (c != 4) c = 3;
+          } else if (at && c != 4) {
+            const long long s1 = c < 3 ? cs.delta[c] : 0;
+            const int n1 = c < 3 ? c + 1 : c;
+            const long long s2 = n1 < 3 ? cs.delta[n1] : 0;
+            const int n2 = n1 < 3 ? n1 + 1 : n1;
+            c = rem <= s1 ? n1 : rem <= s1 + s2 ? n2 : 3;
+          }
+        } else if (before || at) {
+          if (c != 4) ++ev;
+          c = 4;
         }
-      } else if (before || at) {
-        if (c != 4) ++ev;
-        c = 4;
       }
-      if (c != c0) codes[i] = (int8_t)c;
+      o[e] = c;
+      if (i + e < n && c >= 0 && c <= 4) bytes += (unsigned long long)cs.cost[c];
+      if (next && elig) {
+        const unsigned long long w = weight(cs, MODE_EVICT, c);
+        if (w != 0) atomicAdd(&lh[digit_of(k, 0)], w);
+      }
     }
-    if (c >= 0 && c <= 4) bytes += (unsigned long long)cs.cost[c];
+    store4(out, i, n, o);
   }
+  if (next) flush_hist(lh, hist + 3 * MODE_EVICT * BINS);
   bytes = block_sum(bytes, red);
   ev = block_sum(ev, red);
   if (threadIdx.x == 0) {
-    atomicAdd(&st->pred[slot], bytes);
-    if (ev) atomicAdd(&st->evicted, ev);
+    unsigned long long* r = reinterpret_cast<unsigned long long*>(result);
+    atomicAdd(next ? &st->pred[1] : r, bytes);
+    if (ev) atomicAdd(r + 1, ev);  // evictions only in the last pass
   }
-}
-
-__global__ void adm_finish(const AdmState* st, int64_t* result) {
-  if (threadIdx.x != 0) return;
-  result[0] = (int64_t)st->pred[2];
-  result[1] = (int64_t)st->evicted;
-  result[2] = st->bad;
 }
 
 // ---- kv_sensitivity ----------------------------------------------------------
@@ -414,23 +539,25 @@ namespace {
 size_t adm_align(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct AdmLayout {
-  size_t key, cand, hist, blk, state, total;
+  size_t key, cand, mid, hist, blk, state, total;
 };
 
 AdmLayout adm_layout(int64_t n) {
   AdmLayout l;
   const int64_t nblk = ceil_div(n, TIE_CHUNK);
+  const size_t n4 = ((size_t)n + 3) & ~(size_t)3;
   l.key = 0;
-  l.cand = adm_align(l.key + (size_t)n * 4);
-  l.hist = adm_align(l.cand + (size_t)n);
-  l.blk = adm_align(l.hist + 256 * 8);
+  l.cand = adm_align(l.key + n4 * 4);
+  l.mid = adm_align(l.cand + n4);  // the codes after the downgrade
+  l.hist = adm_align(l.mid + (size_t)n);
+  l.blk = adm_align(l.hist + 6 * BINS * 8);
   l.state = adm_align(l.blk + (size_t)(nblk > 0 ? nblk : 1) * 8);
   l.total = adm_align(l.state + sizeof(AdmState));
   return l;
 }
 
 unsigned adm_grid(int64_t n) {
-  return (unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, ADM_THREADS), 2048));
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, 4 * ADM_THREADS), kAdmBlocks));
 }
 
 }  // namespace
@@ -470,28 +597,31 @@ extern "C" int si_admit_codes(const int8_t* codes, int8_t* out_codes, int64_t S,
   for (int c = 0; c < 5; ++c) cs.cost[c] = costs[c];
   for (int c = 0; c < 3; ++c) cs.delta[c] = costs[c] - costs[c + 1];
 
-  adm_init<<<1, 256, 0, st>>>(state, hist, budget_bytes, use_budget ? 1 : 0);
+  int8_t* mid = reinterpret_cast<int8_t*>(ws + l.mid);
+  adm_init<<<1, ADM_THREADS, 0, st>>>(state, hist, budget_bytes, result);
   if (int rc = check_launch("si_admit_codes")) return rc;
-  if (n > 0) {
-    const unsigned grid = adm_grid(n);
-    const int64_t nblk = ceil_div(n, TIE_CHUNK);
-    adm_prep<<<grid, ADM_THREADS, 0, st>>>(codes, out_codes, n, H, importance, sensitivity,
-                                           protected_mask, sink_tokens, cs, key, cand, state);
-    for (int mode = MODE_DOWN; mode <= MODE_EVICT; ++mode) {
-      adm_sel_begin<<<1, 64, 0, st>>>(state, mode, allow_eviction);
-      for (int d = 3; d >= 0; --d) {
-        adm_hist<<<grid, ADM_THREADS, 0, st>>>(mode, d, key, cand, out_codes, n, cs, hist, state);
-        adm_pick<<<1, 256, 0, st>>>(d, hist, state);
-      }
-      adm_tie_sum<<<(unsigned)nblk, ADM_THREADS, 0, st>>>(mode, key, cand, out_codes, n, cs, blk,
-                                                           state);
-      adm_tie_pick<<<1, 1024, 0, st>>>(mode, key, cand, out_codes, n, cs, blk, nblk, state);
-      adm_apply<<<grid, ADM_THREADS, 0, st>>>(mode, key, cand, out_codes, n, cs, state,
-                                              mode == MODE_DOWN ? 1 : 2);
-    }
-    if (int rc = check_launch("si_admit_codes")) return rc;
+  if (n == 0) return SI_OK;
+  const unsigned grid = adm_grid(n);
+  const int64_t nblk = ceil_div(n, TIE_CHUNK);
+  SI_CHECK_ARG(nblk < ((int64_t)1 << 31), "si_admit_codes: too many entries (%lld)", (long long)n);
+  // entries before `first` belong to sink tokens
+  const int64_t first = std::max<int64_t>(0, std::min(sink_tokens, S)) * H;
+  adm_prep<<<grid, ADM_THREADS, 0, st>>>(codes, use_budget ? nullptr : out_codes, n, first,
+                                         importance, sensitivity, protected_mask, cs, key, cand,
+                                         hist, state, result);
+  if (int rc = check_launch("si_admit_codes")) return rc;
+  if (!use_budget) return SI_OK;
+  // Each pass reads one code array and writes another: every block of adm_apply
+  // reads the cut entry's chunk, which others would be rewriting.
+  for (int mode = MODE_DOWN; mode <= (allow_eviction ? MODE_EVICT : MODE_DOWN); ++mode) {
+    const int8_t* from = mode == MODE_DOWN ? codes : mid;
+    const bool last = mode == MODE_EVICT || !allow_eviction;
+    for (int d = 1; d <= 2; ++d)
+      adm_hist<<<grid, ADM_THREADS, 0, st>>>(mode, d, key, cand, from, n, cs, hist, state);
+    adm_tie<<<(unsigned)nblk, ADM_THREADS, 0, st>>>(mode, key, cand, from, n, cs, hist, blk, state);
+    adm_apply<<<grid, ADM_THREADS, 0, st>>>(mode, key, cand, from, last ? out_codes : mid, n, cs,
+                                            hist, blk, nblk, state, last ? result : nullptr);
   }
-  adm_finish<<<1, 64, 0, st>>>(state, result);
   return check_launch("si_admit_codes");
 }
 

@@ -370,6 +370,13 @@ extern "C" int si_plan_scan(const int8_t* codes, const uint8_t* evict_mask, int6
     plan_count<<<dim3((unsigned)ntiles), dim3(kThreads), 0, st>>>(codes, evict_mask, n,
                                                                   tile_counts);
     if (int rc = check_launch("si_plan_scan/count")) return rc;
+    if (ntiles <= kFusedMaxTiles) {
+      // each block adds up the tiles before it: one launch fewer before the
+      // caller reads the counts (8192 x 32: 9.2 -> 8.3 us of kernels)
+      plan_slots_lists<<<dim3((unsigned)ntiles), dim3(kThreads), 0, st>>>(
+          codes, evict_mask, 1, n, tile_counts, out_code, out_slot, out_counts, ListsOut{});
+      return check_launch("si_plan_scan/slots");
+    }
   }
   plan_offsets<<<1, kThreads, 0, st>>>(tile_counts, n > 0 ? ntiles : 0, n, tile_base,
                                        out_counts);

@@ -277,3 +277,26 @@ def test_hip_predict_and_guards(dev):
     out, pred, ev = admit_codes(empty, torch.zeros(0, 4), torch.zeros(0, 4), 0, 1, 16,
                                 allow_eviction=True)
     assert out.shape == (0, 4) and (pred, ev) == (0, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,H,skip", [(1365, 3, 1), (4099, 1, 3), (65537, 5, 0), (2049, 1031, 0)])
+def test_hip_admit_codes_chunk_edges_and_ties(dev, S, H, skip):
+    """Entry counts around the groups of four, the 2048-entry tie chunks and, with
+    2.1 M entries, more chunks than a block scans at once; almost all scores tie,
+    so the cut is found by index; code rows at odd addresses."""
+    rng = np.random.default_rng(S)
+    B, D = 1, 64
+    codes = rng.integers(0, 4, size=(S + skip, H)).astype(np.int8)
+    imp = np.full((S, H), 0.5, np.float32)
+    imp[rng.random((S, H)) < 0.01] = 0.25
+    sens = np.ones((S, H), np.float32)
+    total = int(O.code_costs(B, D)[codes[skip:].astype(np.int64)].sum())
+    dev_codes = torch.from_numpy(codes).to(dev)[skip:]
+    from shadowinfer_amd.shadowkv import admit_codes
+    for budget, evict in ((total - 777, False), (total * 2 // 3, False), (total // 7, True)):
+        want = O.admit_codes(codes[skip:], imp, sens, budget, B, D, 1, True, evict)
+        out, pred, ev = admit_codes(dev_codes, torch.from_numpy(imp), torch.from_numpy(sens), budget,
+                                    B, D, 1, True, evict)
+        np.testing.assert_array_equal(out.cpu().numpy(), want[0])
+        assert (pred, ev) == want[1:]
