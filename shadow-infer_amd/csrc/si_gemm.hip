@@ -79,6 +79,39 @@ __device__ __forceinline__ void store_dequant(const EpiArgs& ep, int64_t idx, in
   store_any(ep.out, ep.out_dtype, idx, add_resid_rt(ep, idx, o));
 }
 
+// store_dequant of four consecutive columns (idx a multiple of 4, ep.vec set).
+__device__ __forceinline__ void store4_dequant(const EpiArgs& ep, int64_t idx, const int32_t (&v)[4],
+                                               float sx, const float (&w)[4], const float (&bb)[4]) {
+  float o[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    o[j] = (float)v[j] * (sx * w[j]);
+    if (ep.bias != nullptr) o[j] = o[j] + bb[j];
+  }
+  if (ep.out_dtype == SI_DT_F32) {
+    float* out = reinterpret_cast<float*>(ep.out) + idx;
+    if (ep.resid != nullptr) {
+      const float4 r = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(ep.resid) + idx);
+      o[0] += r.x; o[1] += r.y; o[2] += r.z; o[3] += r.w;
+    }
+    *reinterpret_cast<float4*>(out) = make_float4(o[0], o[1], o[2], o[3]);
+    return;
+  }
+  const bool f16 = ep.out_dtype == SI_DT_F16;
+  if (ep.resid != nullptr) {
+    const uint2 r = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(ep.resid) + idx);
+    const uint32_t rh[4] = {r.x & 0xffffu, r.x >> 16, r.y & 0xffffu, r.y >> 16};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[j] = round_to(o[j], ep.out_dtype) + (f16 ? f16_bits_to_f32(rh[j]) : bf16_bits_to_f32(rh[j]));
+  }
+  uint32_t h[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) h[j] = f16 ? f32_to_f16_bits(o[j]) : f32_to_bf16_bits(o[j]);
+  *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(ep.out) + idx) =
+      make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+}
+
 template <int EPI>
 __device__ __forceinline__ void epi_store(const EpiArgs& ep, int32_t* C, int64_t M, int64_t N,
                                           int64_t m, int64_t n, int32_t v, int split) {
@@ -1164,34 +1197,7 @@ __global__ __launch_bounds__(256) void gemm_rows(const int8_t* __restrict__ A,
     }
     const float w[4] = {esw[x].x, esw[x].y, esw[x].z, esw[x].w};
     const float bb[4] = {eb[x].x, eb[x].y, eb[x].z, eb[x].w};
-    float o[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      o[j] = (float)v[j] * (esx[x] * w[j]);
-      if (ep.bias != nullptr) o[j] = o[j] + bb[j];
-    }
-    if (ep.out_dtype == SI_DT_F32) {
-      float* out = reinterpret_cast<float*>(ep.out) + idx;
-      if (ep.resid != nullptr) {
-        const float4 r = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(ep.resid) + idx);
-        o[0] += r.x; o[1] += r.y; o[2] += r.z; o[3] += r.w;
-      }
-      *reinterpret_cast<float4*>(out) = make_float4(o[0], o[1], o[2], o[3]);
-    } else {
-      const bool f16 = ep.out_dtype == SI_DT_F16;
-      if (ep.resid != nullptr) {
-        const uint2 r = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(ep.resid) + idx);
-        const uint32_t rh[4] = {r.x & 0xffffu, r.x >> 16, r.y & 0xffffu, r.y >> 16};
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          o[j] = round_to(o[j], ep.out_dtype) + (f16 ? f16_bits_to_f32(rh[j]) : bf16_bits_to_f32(rh[j]));
-      }
-      uint32_t h[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) h[j] = f16 ? f32_to_f16_bits(o[j]) : f32_to_bf16_bits(o[j]);
-      *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(ep.out) + idx) =
-          make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-    }
+    store4_dequant(ep, idx, v, esx[x], w, bb);
   }
 }
 
@@ -1212,6 +1218,41 @@ __global__ __launch_bounds__(256) void gemm_finalize(const int32_t* __restrict__
       const int64_t n = i - m * N;
       store_dequant(ep, i, acc, ep.sx[m], ep.sw[n], ep.bias != nullptr ? ep.bias[n] : 0.0f);
     }
+  }
+}
+
+// The same for four columns per thread, 16-byte loads and the partials of up to
+// four splits in flight (N % 8 == 0, every pointer aligned: ep.vec). 512 x 4096 in
+// four splits, bf16 out: 12.0 -> 4.8 us (38 MB); 77 x 4096 fp32 stays at 4.0 (launch).
+__global__ __launch_bounds__(256) void gemm_finalize4(const int32_t* __restrict__ partial,
+                                                      int splits, int64_t M, int64_t N,
+                                                      int32_t* __restrict__ C, EpiArgs ep,
+                                                      int dequant) {
+  const int64_t total = M * N, n4 = N / 4;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total / 4;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    v4i acc = {0, 0, 0, 0};
+    for (int s0 = 0; s0 < splits; s0 += 4) {
+      v4i p[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        p[u] = v4i{0, 0, 0, 0};
+        if (s0 + u < splits)
+          p[u] = *reinterpret_cast<const v4i*>(partial + (int64_t)(s0 + u) * total + 4 * i);
+      }
+      acc += (p[0] + p[1]) + (p[2] + p[3]);
+    }
+    if (!dequant) {
+      *reinterpret_cast<v4i*>(C + 4 * i) = acc;
+      continue;
+    }
+    const int64_t m = i / n4, n = 4 * (i - m * n4);
+    const float4 w = *reinterpret_cast<const float4*>(ep.sw + n);
+    float4 b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (ep.bias != nullptr) b = *reinterpret_cast<const float4*>(ep.bias + n);
+    const int32_t v[4] = {acc[0], acc[1], acc[2], acc[3]};
+    const float ws[4] = {w.x, w.y, w.z, w.w}, bb[4] = {b.x, b.y, b.z, b.w};
+    store4_dequant(ep, 4 * i, v, ep.sx[m], ws, bb);
   }
 }
 
@@ -1590,19 +1631,21 @@ void launch(const Plan& p, const int8_t* a, const int8_t* b, int M, int N, int K
   }
 }
 
+// Whether the epilogues may use whole 16-byte pieces. The int32 epilogues'
+// device-scope buffer stores address a band of at most 128 output rows by a
+// 32-bit byte offset (< 512 N): wider outputs take the per-element stores.
+int epi_vec(const EpiArgs& ep, const int32_t* c, const void* ws, int64_t N) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(ep.out) |
+                         reinterpret_cast<uintptr_t>(ep.sw) | reinterpret_cast<uintptr_t>(ep.bias) |
+                         reinterpret_cast<uintptr_t>(ep.resid) | reinterpret_cast<uintptr_t>(ws);
+  return (N % 8 == 0 && (bits & 15) == 0 && N < ((int64_t)1 << 22)) ? 1 : 0;
+}
+
 int run_gemm(const int8_t* a, const int8_t* b, int64_t M, int64_t N, int64_t K, int32_t* c,
              EpiArgs ep, bool dequant, void* ws, size_t ws_bytes, hipStream_t st, const char* who) {
   if (M == 0 || N == 0) return SI_OK;
   const Plan p = choose(M, N, K);
-  {
-    uintptr_t bits = reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(ep.out) |
-                     reinterpret_cast<uintptr_t>(ep.sw) | reinterpret_cast<uintptr_t>(ep.bias) |
-                     reinterpret_cast<uintptr_t>(ep.resid) | reinterpret_cast<uintptr_t>(ws);
-    // The int32 epilogues' device-scope buffer stores address a band of at
-    // most 128 output rows by a 32-bit byte offset (< 512 N): wider outputs
-    // take the per-element stores.
-    ep.vec = (N % 8 == 0 && (bits & 15) == 0 && N < ((int64_t)1 << 22)) ? 1 : 0;
-  }
+  ep.vec = epi_vec(ep, c, ws, N);
   if (p.kind == K_SCALAR) {
     const int64_t blocks = std::min<int64_t>(ceil_div(M * N, 256), 65536);
     gemm_i8_scalar<<<(unsigned)blocks, 256, 0, st>>>(a, b, M, N, K, c, ep, dequant ? 1 : 0);
@@ -1626,6 +1669,12 @@ int run_gemm(const int8_t* a, const int8_t* b, int64_t M, int64_t N, int64_t K, 
   ep.partial = reinterpret_cast<int32_t*>(ws);
   launch<EPI_PARTIAL>(p, a, b, Mi, Ni, Ki, c, ep, st);
   if (int rc = check_launch(who)) return rc;
+  if (ep.vec) {
+    const int64_t blocks = std::min<int64_t>(ceil_div(M * N / 4, 256), 65536);
+    gemm_finalize4<<<(unsigned)blocks, 256, 0, st>>>(ep.partial, p.splits, M, N, c, ep,
+                                                    dequant ? 1 : 0);
+    return check_launch(who);
+  }
   const int64_t blocks = std::min<int64_t>(ceil_div(M * N, 256), 65536);
   gemm_finalize<<<(unsigned)blocks, 256, 0, st>>>(ep.partial, p.splits, M, N, c, ep,
                                                  dequant ? 1 : 0);
