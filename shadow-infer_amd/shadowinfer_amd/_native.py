@@ -181,7 +181,7 @@ def _refuse_forced_cpu(what: str) -> None:
 def call(name: str, *args) -> None:
     """Invoke ``name`` and raise RuntimeError with the library's message on failure."""
     _refuse_forced_cpu(name)
-    lib = load()
+    lib = _lib or load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         msg = lib.si_last_error().decode(errors="replace")
@@ -191,7 +191,7 @@ def call(name: str, *args) -> None:
 
 
 def size_query(name: str, *args) -> int:
-    return int(getattr(load(), name)(*args))
+    return getattr(_lib or load(), name)(*args)
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -199,7 +199,10 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of torch's current stream on ``device``, without the Stream
+    object around it (0.3 instead of 3.5 us a call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -224,14 +227,8 @@ def require_device(t: torch.Tensor, what: str) -> None:
 
 
 def table16(ptrs) -> "ctypes.Array":
-    arr = _PTR16()
-    for i, p in enumerate(ptrs):
-        arr[i] = p
-    return arr
+    return _PTR16(*ptrs)
 
 
 def table4(ptrs) -> "ctypes.Array":
-    arr = _PTR4()
-    for i, p in enumerate(ptrs):
-        arr[i] = p
-    return arr
+    return _PTR4(*ptrs)

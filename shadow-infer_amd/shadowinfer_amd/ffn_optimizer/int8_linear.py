@@ -132,24 +132,25 @@ class INT8Linear(nn.Module):
         """int8_linear.py:88-115."""
         if x.shape[-1] != self.in_features:
             raise ValueError(f"input last dim {x.shape[-1]} != in_features {self.in_features}")
-        leading_shape = x.shape[:-1]
-        flat = x.reshape(-1, self.in_features)
+        K, N = self.in_features, self.out_features
+        flat = x if x.dim() == 2 else x.reshape(-1, K)
+        dev = x.device
         if flat.numel() == 0:
-            return torch.empty((*leading_shape, self.out_features), dtype=x.dtype, device=x.device)
+            return torch.empty((*x.shape[:-1], N), dtype=x.dtype, device=dev)
         _native.require_device(flat, "INT8Linear.forward")
-        if self.qweight_nk.device != flat.device:
-            raise ValueError(f"input on {flat.device} but weights on {self.qweight_nk.device}")
-        dt = _native.dtype_code(flat.dtype)
+        weight = self.qweight_nk
+        if weight.device != dev:
+            raise ValueError(f"input on {dev} but weights on {weight.device}")
+        dt = _native.dtype_code(x.dtype)
         flat = flat.contiguous()
-        M, K, N = flat.shape[0], self.in_features, self.out_features
-        out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        M = flat.shape[0]
+        out = torch.empty((M, N), dtype=x.dtype, device=dev)
         ws_bytes = _native.size_query("si_int8_linear_workspace_bytes", M, K, N)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-        _native.call("si_int8_linear_forward", flat.data_ptr(), dt, M, K, N,
-                     self.qweight_nk.data_ptr(), self.weight_scale.data_ptr(),
-                     _native.ptr(self.bias), out.data_ptr(), ws.data_ptr(), ws_bytes,
-                     _native.stream(x.device))
-        return out.reshape(*leading_shape, N)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        _native.call("si_int8_linear_forward", flat.data_ptr(), dt, M, K, N, weight.data_ptr(),
+                     self.weight_scale.data_ptr(), _native.ptr(self.bias), out.data_ptr(),
+                     ws.data_ptr(), ws_bytes, _native.stream(dev))
+        return out if x.dim() == 2 else out.reshape(*x.shape[:-1], N)
 
     def memory_bytes(self) -> int:
         """Bytes held: the int8 weight, fp32 scales and fp32 bias

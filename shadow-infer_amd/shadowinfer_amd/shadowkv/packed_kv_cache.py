@@ -65,8 +65,8 @@ class PackedKVCache:
         cache = cls(batch_size, num_heads, seq_len, head_dim, device=k_tensor.device)
         cache._do_pack(k_tensor, v_tensor, precision_map, group_size=group_size, plan=plan,
                        precomputed=precomputed)
-        return {"packed_kv": cache, "memory_bytes": cache.memory_bytes(),
-                "memory_mb": cache.memory_mb()}
+        total = cache.memory_bytes()
+        return {"packed_kv": cache, "memory_bytes": total, "memory_mb": total / (1024.0 * 1024.0)}
 
     @classmethod
     def pack_projection(cls, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
@@ -97,14 +97,13 @@ class PackedKVCache:
         cache._scale_dtype = qkv.dtype
         cache._buckets = cache._alloc_buckets(grouping.counts, dev, qkv.dtype)
         cache._view = None
-        flat = grouping.flat_lists(S, H)
-        counts = (ctypes.c_int64 * 5)(*[int(c) for c in grouping.counts])
+        flat, counts = grouping.list_tables(S, H)
         # contiguous copies stay bound until the launch is queued
         src, cos_c, sin_c = qkv.contiguous(), cos.contiguous(), sin.contiguous()
         _native.call("si_kv_pack_rope_flat", src.data_ptr(), cos_c.data_ptr(), sin_c.data_ptr(),
                      _native.dtype_code(qkv.dtype), B, H, S, D, g, grouping.code.data_ptr(),
-                     grouping.slot.data_ptr(), _native.table4([f.data_ptr() for f in flat]),
-                     counts, cache._bucket_table(), _native.stream(dev))
+                     grouping.slot.data_ptr(), flat, counts, cache._bucket_table(),
+                     _native.stream(dev))
         return cache
 
     def _do_pack(self, k_tensor: torch.Tensor, v_tensor: torch.Tensor,
@@ -156,11 +155,9 @@ class PackedKVCache:
         self._buckets = self._alloc_buckets(grouping.counts, dev, k.dtype)
         self._view = None
         if work_copy is None:
-            flat = grouping.flat_lists(S, H)
-            counts = (ctypes.c_int64 * 5)(*[int(c) for c in grouping.counts])
+            flat, counts = grouping.list_tables(S, H)
             _native.call("si_kv_pack_flat", k.data_ptr(), v.data_ptr(), dt, B, H, S, D, g,
-                         grouping.code.data_ptr(), grouping.slot.data_ptr(),
-                         _native.table4([f.data_ptr() for f in flat]), counts,
+                         grouping.code.data_ptr(), grouping.slot.data_ptr(), flat, counts,
                          self._bucket_table(), _native.stream(dev))
         else:
             out_k, out_v, k_prev, v_prev, reuse = work_copy
@@ -203,10 +200,10 @@ class PackedKVCache:
         buckets = self._buckets if buckets is None else buckets
         ptrs: List[Optional[int]] = [None] * 16
         for name, data in buckets.items():
-            p = _PREC_INDEX[name]
-            for j, key in enumerate(("k", "v", "scale_k", "scale_v")):
-                t = data.get(key)
-                ptrs[4 * p + j] = None if t is None else t.data_ptr()
+            p = 4 * _PREC_INDEX[name]
+            ptrs[p], ptrs[p + 1] = data["k"].data_ptr(), data["v"].data_ptr()
+            if data["scale_k"] is not None:
+                ptrs[p + 2], ptrs[p + 3] = data["scale_k"].data_ptr(), data["scale_v"].data_ptr()
         return _native.table16(ptrs)
 
     def _apply_precomputed(self, precomputed: Dict[str, Any], counts: List[int]) -> None:
@@ -255,10 +252,8 @@ class PackedKVCache:
         v_out = torch.empty(shape, dtype=torch.float32, device=dev)
         if k_out.numel():
             gr = self._grouping
-            flat = gr.flat_lists(self.seq_len, self.num_heads)
-            counts = (ctypes.c_int64 * 5)(*[int(c) for c in gr.counts])
-            _native.call("si_kv_unpack_flat", gr.code.data_ptr(), gr.slot.data_ptr(),
-                         _native.table4([f.data_ptr() for f in flat]), counts,
+            flat, counts = gr.list_tables(self.seq_len, self.num_heads)
+            _native.call("si_kv_unpack_flat", gr.code.data_ptr(), gr.slot.data_ptr(), flat, counts,
                          self._bucket_table(), _native.dtype_code(self._scale_dtype), *shape,
                          self._group_size, k_out.data_ptr(), v_out.data_ptr(),
                          _native.stream(dev))
@@ -306,10 +301,9 @@ class PackedKVCache:
     def _compute_data_bytes(self) -> int:
         total = 0
         for data in self._buckets.values():
-            for key in ("k", "v", "scale_k", "scale_v"):
-                t = data.get(key)
-                if t is not None:
-                    total += t.numel() * t.element_size()
+            total += data["k"].nbytes + data["v"].nbytes
+            if data["scale_k"] is not None:
+                total += data["scale_k"].nbytes + data["scale_v"].nbytes
         return total
 
     def data_plane_bytes(self) -> int:
@@ -355,20 +349,15 @@ class PackedKVCache:
         if removed == 0:
             return 0
         new_buckets: Dict[str, Dict[str, Any]] = {}
-        changed: Dict[str, Dict[str, Any]] = {}
-        fresh = self._alloc_buckets(counts, dev, self._scale_dtype)
-        for name in PRECISION_ORDER:
-            p = _PREC_INDEX[name]
-            if counts[p] == 0:
-                continue
-            if counts[p] == old.counts[p]:
-                new_buckets[name] = self._buckets[name]  # untouched (reference keeps it)
-            else:
-                new_buckets[name] = fresh[name]
-                changed[name] = fresh[name]
+        # buckets that lose nothing are kept as they are (as in the reference)
+        changed = self._alloc_buckets([c if c != o else 0 for c, o in zip(counts, old.counts)], dev,
+                                      self._scale_dtype)
+        for p, name in enumerate(PRECISION_ORDER):
+            if counts[p]:
+                new_buckets[name] = changed[name] if name in changed else self._buckets[name]
         flat = [torch.empty(c, dtype=torch.long, device=dev) for c in counts[:4]]
-        _native.call("si_kv_evict_flat", _native.table4([f.data_ptr() for f in old.flat_lists(S, H)]),
-                     (ctypes.c_int64 * 4)(*old.counts[:4]), chunk_counts.data_ptr(),
+        old_flat, old_counts = old.list_tables(S, H)
+        _native.call("si_kv_evict_flat", old_flat, old_counts, chunk_counts.data_ptr(),
                      chunk_bits.data_ptr(), S, H, self._bucket_table(), _native.table4([f.data_ptr() for f in flat]),
                      (ctypes.c_int64 * 4)(*counts[:4]), self._bucket_table(changed), slot.data_ptr(),
                      self.batch_size, self.head_dim, self._group_size,
@@ -436,9 +425,8 @@ class PackedKVCache:
             mask = host.to(dev)
         stats_dev = torch.zeros(2, dtype=torch.int64, device=dev) if return_stats else None
         grouping = self._grouping
-        flat = grouping.flat_lists(self.seq_len, self.num_heads)
-        _native.call("si_kv_reuse_flat", _native.table4([f.data_ptr() for f in flat]),
-                     (ctypes.c_int64 * 5)(*grouping.counts), self._bucket_table(), self.seq_len,
+        flat, counts = grouping.list_tables(self.seq_len, self.num_heads)
+        _native.call("si_kv_reuse_flat", flat, counts, self._bucket_table(), self.seq_len,
                      prev._grouping.code.data_ptr(), prev._grouping.slot.data_ptr(),
                      prev._bucket_table(), prev.seq_len, mask.data_ptr(), self.num_heads,
                      self.batch_size, self.head_dim, self._group_size,

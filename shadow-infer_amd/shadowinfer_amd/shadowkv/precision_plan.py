@@ -128,7 +128,7 @@ class DeviceGrouping:
     so what is derived from them stays valid.
     """
 
-    __slots__ = ("code", "slot", "counts", "flat", "attn")
+    __slots__ = ("code", "slot", "counts", "flat", "attn", "_tables")
 
     def __init__(self, code: torch.Tensor, slot: torch.Tensor, counts: List[int],
                  flat: Optional[List[torch.Tensor]] = None):
@@ -137,6 +137,16 @@ class DeviceGrouping:
         self.counts = counts
         self.flat = flat
         self.attn: Optional[torch.Tensor] = None
+        self._tables: Optional[tuple] = None
+
+    def list_tables(self, S: int, H: int) -> tuple:
+        """(pointer table of ``flat``, ``counts`` as C int64) for the C ABI, made
+        once: this grouping holds the lists and neither ever changes."""
+        if self._tables is None:
+            flat = self.flat_lists(S, H)
+            self._tables = (_native.table4([f.data_ptr() for f in flat]),
+                            (ctypes.c_int64 * 5)(*self.counts))
+        return self._tables
 
     def attn_lists(self, S: int, H: int) -> torch.Tensor:
         """Per-head slot lists of the fused attention (si_attn_build_lists)."""
@@ -174,7 +184,7 @@ class DeviceGrouping:
         _native.call("si_plan_scan", codes_flat.data_ptr(),
                      _native.ptr(evict_mask), n, code.data_ptr(), slot.data_ptr(),
                      counts.data_ptr(), ws.data_ptr(), ws_bytes, _native.stream(dev))
-        return DeviceGrouping(code, slot, [int(c) for c in counts.tolist()])
+        return DeviceGrouping(code, slot, counts.tolist())
 
     def evict_count(self, evict_mask: torch.Tensor, S: int, H: int):
         """First pass of an evict (si_kv_evict_count) over this grouping's
@@ -184,9 +194,8 @@ class DeviceGrouping:
         read from those counts."""
         dev = self.code.device
         n = S * H
-        flat = self.flat_lists(S, H)
+        flat, old = self.list_tables(S, H)
         lib = _native.load()
-        old = (ctypes.c_int64 * 4)(*self.counts[:4])
         chunks = int(lib.si_kv_evict_chunks(old))
         words = int(lib.si_kv_evict_chunk_words())
         code = torch.empty(n, dtype=torch.int8, device=dev)
@@ -194,7 +203,7 @@ class DeviceGrouping:
         cc = torch.empty(max(chunks, 1), dtype=torch.int32, device=dev)
         bits = torch.empty(max(chunks * words, 1), dtype=torch.int64, device=dev)
         _native.call("si_kv_evict_count", self.code.data_ptr(),
-                     _native.table4([f.data_ptr() for f in flat]), old, evict_mask.data_ptr(), S, H,
+                     flat, old, evict_mask.data_ptr(), S, H,
                      code.data_ptr(), slot.data_ptr(), cc.data_ptr(), bits.data_ptr(),
                      _native.stream(dev))
         per = cc[:chunks].cpu().numpy().astype(np.int64)
