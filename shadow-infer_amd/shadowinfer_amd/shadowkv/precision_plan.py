@@ -128,7 +128,7 @@ class DeviceGrouping:
     so what is derived from them stays valid.
     """
 
-    __slots__ = ("code", "slot", "counts", "flat", "attn", "_tables")
+    __slots__ = ("code", "slot", "counts", "flat", "attn")
 
     def __init__(self, code: torch.Tensor, slot: torch.Tensor, counts: List[int],
                  flat: Optional[List[torch.Tensor]] = None):
@@ -137,16 +137,12 @@ class DeviceGrouping:
         self.counts = counts
         self.flat = flat
         self.attn: Optional[torch.Tensor] = None
-        self._tables: Optional[tuple] = None
 
     def list_tables(self, S: int, H: int) -> tuple:
-        """(pointer table of ``flat``, ``counts`` as C int64) for the C ABI, made
-        once: this grouping holds the lists and neither ever changes."""
-        if self._tables is None:
-            flat = self.flat_lists(S, H)
-            self._tables = (_native.table4([f.data_ptr() for f in flat]),
-                            (ctypes.c_int64 * 5)(*self.counts))
-        return self._tables
+        """(pointer table of ``flat``, ``counts`` as C int64) of one call of the C
+        ABI. Made per call: the grouping stays picklable and holds no address."""
+        return (_native.table4([f.data_ptr() for f in self.flat_lists(S, H)]),
+                (ctypes.c_int64 * 5)(*self.counts))
 
     def attn_lists(self, S: int, H: int) -> torch.Tensor:
         """Per-head slot lists of the fused attention (si_attn_build_lists)."""

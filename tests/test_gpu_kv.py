@@ -559,3 +559,17 @@ def test_rows_of_any_chunk_count_bit_exact(dev, dtype, B, H, S, D, g):
     k_out, v_out = cache.unpack()
     np.testing.assert_array_equal(k_out.cpu().numpy(), rk)
     np.testing.assert_array_equal(v_out.cpu().numpy(), rv)
+
+
+@pytest.mark.gpu
+def test_plan_grouping_survives_pickle(dev):
+    """A device plan that has been packed with is saved and loaded like before its
+    first use: it holds tensors and counts, no addresses."""
+    import pickle
+    from shadowinfer_amd.shadowkv.precision_plan import DeviceGrouping
+    code = torch.randint(0, 5, (7 * 3,), device=dev).to(torch.int8)
+    g = DeviceGrouping.scan(code)
+    g.list_tables(7, 3)
+    h = pickle.loads(pickle.dumps(g))
+    assert h.counts == g.counts and torch.equal(h.slot, g.slot)
+    assert all(torch.equal(a, b) for a, b in zip(h.flat, g.flat))
