@@ -66,6 +66,9 @@ def schedule_round(logits_block: torch.Tensor, masked: torch.Tensor,
         raise ValueError(
             f"confidence_threshold must be within (0, 1], got {confidence_threshold}")
     tokens, confidences = argmax_confidence(logits_block)
+    if masked.shape[1] == 0:
+        raise IndexError("a round needs at least one position per row, got masked of shape "
+                         f"{tuple(masked.shape)}")
     dev = logits_block.device
     mask = masked.to(device=dev, dtype=torch.bool).contiguous()
     unmask = torch.empty_like(mask)

@@ -846,3 +846,17 @@ def test_schedule_rows_nan_ties_and_signs(dev, W):
         ru, rt, rc, rf = _reference_schedule(lg, mk, thr)
         assert torch.equal(d.unmask, ru) and torch.equal(d.progress_fallback, rf)
         assert torch.equal(torch.nan_to_num(d.confidences, nan=2.0), torch.nan_to_num(rc, nan=2.0))
+
+
+@pytest.mark.gpu
+def test_schedule_round_without_positions_or_rows(dev):
+    """No position to decide about is refused (an argmax over nothing); no row at
+    all is an empty round."""
+    from shadowinfer_amd.execution import schedule_round
+    for B in (0, 3):
+        with pytest.raises(IndexError):
+            schedule_round(torch.zeros(B, 0, 24, device=dev),
+                           torch.zeros(B, 0, dtype=torch.bool, device=dev), 0.9)
+    d = schedule_round(torch.zeros(0, 5, 24, device=dev),
+                       torch.zeros(0, 5, dtype=torch.bool, device=dev), 0.9)
+    assert d.unmask.shape == (0, 5) and d.progress_fallback.shape == (0,)
