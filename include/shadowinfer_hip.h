@@ -81,8 +81,9 @@ int si_check_bf16_convert(unsigned long long* counts, si_stream_t stream);
 void si_tune_gemm_plan(int kind, int splits);
 void si_tune_attn_offset64(int on);
 
-/* Test and sweep override of the split of a short attention over workgroups:
- * 0 (the start value) by size, -1 never, n > 0 n parts where it applies. */
+/* Test and sweep override of an attention's kernel and key parts: 0 (the start
+ * value) by size, -1 the 256-query kernel unsplit, n = 1..64 the wave-per-half-tile
+ * kernel in n parts, 64 + n the 256-query kernel in n parts, where they apply. */
 void si_tune_attn_parts(int parts);
 
 /* Thread-local text of the last failure (empty string if none). Replaces the

@@ -448,8 +448,9 @@ __device__ __forceinline__ void load_q(const uint16_t* __restrict__ Q, int64_t b
 // row) and read back row-contiguous: each store instruction writes 64 x 16
 // contiguous bytes of SRB / 16 lanes per row. Row r of the wave is query
 // m0 + r at out + obase0 + r * row_stride (elements); rows at or past Sq are
-// not stored.
-template <int D>
+// not stored. RAW stores the rows of one key part as they are, as fp32 (the
+// launch that adds the parts divides).
+template <int D, bool RAW = false>
 __device__ __forceinline__ void finish_rows(v16f* o, float m_run, float l_run, int n_ev, int col,
                                             int grp, uint8_t* stage, int64_t m0, int64_t Sq,
                                             int64_t obase0, int64_t row_stride, void* O,
@@ -458,8 +459,8 @@ __device__ __forceinline__ void finish_rows(v16f* o, float m_run, float l_run, i
   constexpr int DB = D / 32;
   constexpr int CPR = C::SRB / 16;  // 16-byte chunks per staged row
   const int lane = (grp << 5) | col;
-  l_run = halves_sum(l_run);  // each half summed its own keys
-  if (n_ev > 0) {
+  if constexpr (!RAW) l_run = halves_sum(l_run);  // each half summed its own keys
+  if (!RAW && n_ev > 0) {
     const float m_fin = fmaxf(m_run, 0.0f);
     const float alpha = exp2f(m_run - m_fin);
     l_run = l_run * alpha + (float)n_ev * exp2f(-m_fin);
@@ -468,7 +469,7 @@ __device__ __forceinline__ void finish_rows(v16f* o, float m_run, float l_run, i
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
   }
-  const float inv = 1.0f / l_run;  // rows past Sq may divide by 0: never stored
+  const float inv = RAW ? 1.0f : 1.0f / l_run;  // rows past Sq may divide by 0: never stored
   // Device-scope (sc1) buffer stores from the wave's first row: the rows are
   // written through as they leave, so less dirty output waits in L2 for the
   // end-of-kernel writeback (S=2048 83.5 -> 82.0 us with 50-launch medians
@@ -492,7 +493,7 @@ __device__ __forceinline__ void finish_rows(v16f* o, float m_run, float l_run, i
     }
     __builtin_amdgcn_wave_barrier();
   };
-  if (odt == SI_DT_F32) {
+  if (RAW || odt == SI_DT_F32) {
     constexpr int DPP = C::SRB / 4;  // dims per pass
 #pragma unroll
     for (int pd0 = 0; pd0 < D; pd0 += DPP) {
@@ -568,11 +569,16 @@ struct OutStrides {
 // row addresses are 32-bit byte offsets from the (uniform) buffer base, and
 // the full-rate 24-bit multiply forms them: slots are below 2^23 (n_max * B *
 // D * 4 < 2^31 with B * D >= 64) and every row stride below 2^24.
-template <int D, int SDT, int QDT, bool O32>
+// PART: the grid has nch blocks per 256 queries, each with its own consecutive
+// part of the head's tiles; their rows and (m, l) go to part / part_ml, in the
+// layout that attn_combine adds up. For few query blocks over many keys (see
+// attn_split); a template, so the unsplit kernel keeps its registers.
+template <int D, int SDT, int QDT, bool O32, bool PART = false>
 __global__ __launch_bounds__(512) void attn_packed_fwd(
     const uint16_t* __restrict__ Q, int64_t B, int64_t H, int64_t Sq, int64_t cap,
     const int32_t* __restrict__ counts, const int32_t* __restrict__ lists, Buckets bk, int64_t g,
-    float scale_log2, void* __restrict__ O, int odt, OutStrides os) {
+    float scale_log2, void* __restrict__ O, int odt, OutStrides os, int nch,
+    float* __restrict__ part, float* __restrict__ part_ml) {
   using C = AttnCfg<D>;
   constexpr int KS = D / 16;  // MFMA k-steps over the head dim
   constexpr int DB = D / 32;  // 32-row blocks of O^T
@@ -597,7 +603,8 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
                              nq * (int)(gridDim.y * gridDim.z));
   const int64_t h = (w_id / nq) % (int)gridDim.y;
   const int64_t b = w_id / (nq * (int)gridDim.y);
-  const int64_t m = (int64_t)(w_id % nq) * C::BMQ + wave * 32 + col;
+  const int ch = PART ? w_id % nq % nch : 0;
+  const int64_t m = (int64_t)(PART ? w_id % nq / nch : w_id % nq) * C::BMQ + wave * 32 + col;
 
   // Q^T fragments (B operand of S^T = K Q^T): query m, dims ks*16 + 8*grp + 0..7.
   v8h qf[KS];
@@ -609,7 +616,8 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
   // bounds even when every key of the head is evicted).
   const int32_t* lh = lists + h * cap;
   const int kg = tid / C::DGN;
-  const int4 sl0 = *reinterpret_cast<const int4*>(lh + 4 * kg);
+  int4 sl0;
+  if constexpr (!PART) sl0 = *reinterpret_cast<const int4*>(lh + 4 * kg);
 
   // Tile schedule: the head's list regions in order fp32, fp16, int8, int4.
   const int32_t* cnt = counts + h * 8;
@@ -621,7 +629,24 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
     tstart[p + 1] = tstart[p] + (np[p] + BN - 1) / BN;
   }
   const int n_ev = cnt[4];
-  auto tile_valid = [&](int tt, int p) __attribute__((always_inline)) { return min(BN, np[p] - (tt - tstart[p]) * BN); };
+  // A part owns tiles [t_lo, tstart[4]) after the clamp: phases outside of it are
+  // empty, phase p still counts its keys from its own first tile, pend[p] keys
+  // before the end of the list region.
+  int t_lo = 0, pend[4];
+  if constexpr (PART) {
+    const int64_t T = tstart[4];
+    t_lo = (int)(T * ch / nch);
+    const int t_hi = (int)(T * (ch + 1) / nch);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) pend[p] = np[p] + tstart[p] * BN;
+#pragma unroll
+    for (int p = 0; p < 5; ++p) tstart[p] = min(max(tstart[p], t_lo), t_hi);
+    sl0 = *reinterpret_cast<const int4*>(lh + (int64_t)t_lo * BN + 4 * kg);
+  }
+  auto tile_valid = [&](int tt, int p) __attribute__((always_inline)) {
+    if constexpr (PART) return min(BN, pend[p] - tt * BN);
+    else return min(BN, np[p] - (tt - tstart[p]) * BN);
+  };
 
   // Decode-stage coordinates: keys 4*kg .. 4*kg+3 of the tile, dims d0 .. d0+DPT-1.
   const int dg = tid % C::DGN;
@@ -913,11 +938,11 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
   // the first tstart[q] > 0): tile min(1, its last tile), loaded here.
   int4 sl_n2;
   {
-    const int fl = tstart[1] > 0 ? tstart[1] - 1
-                 : tstart[2] > 0 ? tstart[2] - 1
-                 : tstart[3] > 0 ? tstart[3] - 1
-                                 : max(tstart[4] - 1, 0);
-    sl_n2 = *reinterpret_cast<const int4*>(lh + (int64_t)min(1, fl) * BN + 4 * kg);
+    const int fl = tstart[1] > t_lo ? tstart[1] - 1
+                 : tstart[2] > t_lo ? tstart[2] - 1
+                 : tstart[3] > t_lo ? tstart[3] - 1
+                                    : max(tstart[4] - 1, 0);
+    sl_n2 = *reinterpret_cast<const int4*>(lh + (int64_t)min(t_lo + 1, fl) * BN + 4 * kg);
   }
   // During a phase's last tile, the first tile of the next non-empty phase
   // (precision Q > P, the phase starting at tile tstart[P + 1]) is loaded into
@@ -1006,6 +1031,14 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
   uint8_t* stage = wave < 4 ? reinterpret_cast<uint8_t*>(&Ks[0][0][0]) + wave * C::STAGE
                             : reinterpret_cast<uint8_t*>(&Vs[0][0][0]) + (wave - 4) * C::STAGE;
   const int64_t m0 = m - col;
+  if constexpr (PART) {
+    const int64_t unit = (b * H + h) * ((Sq + 31) / 32) + m0 / 32;
+    const int64_t pr = (unit * nch + ch) * 32;
+    l_run = halves_sum(l_run);
+    if (grp == 0 && m < Sq) *reinterpret_cast<float2*>(part_ml + 2 * (pr + col)) = make_float2(m_run, l_run);
+    finish_rows<D, true>(o, m_run, l_run, 0, col, grp, stage, m0, Sq, pr * D, D, part, SI_DT_F32);
+    return;
+  }
   finish_rows<D>(o, m_run, l_run, n_ev, col, grp, stage, m0, Sq, b * os.b + h * os.h + m0 * os.s,
                  os.s, O, odt);
 }
@@ -1022,7 +1055,7 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
 // the loop) and keeps its own (m, l, O). The waves are added in LDS at the end
 // and, with nch > 1, the parts by attn_combine. Every wave decodes its keys
 // alone, which costs about three times the VALU work per query of the
-// 256-query blocks: attn_parts decides where that pays.
+// 256-query blocks: attn_split decides where that pays.
 //
 // Rows: LPR = D / 8 lanes hold 8 dims each of one key, and lane group j of
 // 64 / LPR takes keys RPL * j .. + RPL - 1 of the half tile, so every load
@@ -1424,25 +1457,21 @@ __global__ __launch_bounds__(64) void attn_combine(const float* __restrict__ par
   short_store<DPT>(acc, M, L, counts[h * 8 + 4], O, b * os.b + h * os.h + m * os.s + d, odt);
 }
 
-template <int D, int QDT, bool O32>
+template <int D, int QDT, bool O32, bool PART>
 void launch_attn_o(int sdt, dim3 grid, hipStream_t st, const uint16_t* q, int64_t B, int64_t H,
                    int64_t Sq, int64_t cap, const int32_t* counts, const int32_t* lists,
                    const Buckets& bk, int64_t g, float scale_log2, void* out, int odt,
-                   const OutStrides& os) {
+                   const OutStrides& os, int nch, float* part, float* ml) {
   constexpr int NT = 64 * AttnCfg<D>::NW;
+#define SI_FULL(SDT_)                                                                              \
+  attn_packed_fwd<D, SDT_, QDT, O32, PART><<<grid, NT, 0, st>>>(q, B, H, Sq, cap, counts, lists, bk, \
+                                                          g, scale_log2, out, odt, os, nch, part, ml)
   switch (sdt) {
-    case SI_DT_F32:
-      attn_packed_fwd<D, SI_DT_F32, QDT, O32><<<grid, NT, 0, st>>>(q, B, H, Sq, cap, counts, lists,
-                                                                   bk, g, scale_log2, out, odt, os);
-      break;
-    case SI_DT_F16:
-      attn_packed_fwd<D, SI_DT_F16, QDT, O32><<<grid, NT, 0, st>>>(q, B, H, Sq, cap, counts, lists,
-                                                                   bk, g, scale_log2, out, odt, os);
-      break;
-    default:
-      attn_packed_fwd<D, SI_DT_BF16, QDT, O32><<<grid, NT, 0, st>>>(q, B, H, Sq, cap, counts, lists,
-                                                                    bk, g, scale_log2, out, odt, os);
+    case SI_DT_F32: SI_FULL(SI_DT_F32); break;
+    case SI_DT_F16: SI_FULL(SI_DT_F16); break;
+    default: SI_FULL(SI_DT_BF16);
   }
+#undef SI_FULL
 }
 
 // Set by si_tune_attn_offset64 (tests): 64-bit addressing at every size.
@@ -1457,56 +1486,82 @@ bool offsets32(int64_t n_max, int64_t B, int64_t D) {
          !g_force_offset64.load(std::memory_order_relaxed);
 }
 
+// nch > 1 (32-bit offsets only): key parts, added up by a second launch.
 template <int D, int QDT>
 void launch_attn(int sdt, dim3 grid, hipStream_t st, const uint16_t* q, int64_t B, int64_t H,
                  int64_t Sq, int64_t cap, const int32_t* counts, const int32_t* lists,
                  const Buckets& bk, int64_t g, float scale_log2, void* out, int odt,
-                 const OutStrides& os, int64_t n_max) {
-  if (offsets32(n_max, B, D))
-    launch_attn_o<D, QDT, true>(sdt, grid, st, q, B, H, Sq, cap, counts, lists, bk, g, scale_log2,
-                                out, odt, os);
-  else
-    launch_attn_o<D, QDT, false>(sdt, grid, st, q, B, H, Sq, cap, counts, lists, bk, g, scale_log2,
-                                 out, odt, os);
+                 const OutStrides& os, bool o32, int nch, void* ws) {
+  if (nch > 1) {
+    const int nq = (int)ceil_div(Sq, 32);
+    const int64_t units = (int64_t)nq * H * B;
+    float* part = reinterpret_cast<float*>(ws);
+    float* ml = part + units * nch * 32 * D;
+    grid.x *= (unsigned)nch;
+    launch_attn_o<D, QDT, true, true>(sdt, grid, st, q, B, H, Sq, cap, counts, lists, bk, g,
+                                      scale_log2, out, odt, os, nch, part, ml);
+    attn_combine<D><<<(unsigned)(units * 8), 64, 0, st>>>(part, ml, nch, nq, H, Sq, counts, out, odt, os);
+  } else if (o32) {
+    launch_attn_o<D, QDT, true, false>(sdt, grid, st, q, B, H, Sq, cap, counts, lists, bk, g,
+                                       scale_log2, out, odt, os, 1, nullptr, nullptr);
+  } else {
+    launch_attn_o<D, QDT, false, false>(sdt, grid, st, q, B, H, Sq, cap, counts, lists, bk, g,
+                                        scale_log2, out, odt, os, 1, nullptr, nullptr);
+  }
 }
 
-// Parts of attn_packed_short for a call, 0 for attn_packed_fwd (see run_attn for
-// what the short kernel asks of the buffers). Set by si_tune_attn_parts (tests
-// and sweeps): 0 automatic, -1 never the short kernel, n > 0 that many parts.
+// Kernel and key parts of a call. Set by si_tune_attn_parts (tests and sweeps):
+// 0 automatic, -1 attn_packed_fwd in one part, n = 1..64 attn_packed_short in
+// that many parts, 64 + n attn_packed_fwd in n.
 std::atomic<int> g_force_parts{0};
 
-//
-// The rule compares two time estimates (us), fitted on S_kv = 100..8192, H = 4..32:
+// The rule compares time estimates (us), fitted on S_kv = 100..8192, H = 4..32:
 // attn_packed_fwd takes 9 + 1.6 per 64-key tile and round of 256 blocks (D = 64:
-// 1.2; 2.0 where its blocks fill over half the chip, as the clock then drops),
+// 1.1; a quarter more where its blocks fill over 160 CUs, as the clock then drops),
 // the short kernel 6 + 2.15 per half tile and wave (D = 64: 1.3) and, with n > 1
-// parts, 3.5 for the second launch and the partial rows at 3 TB/s; caches of fp32
-// inputs pay for the low parts of K. Measured (D = 128 unless stated, bf16 caches,
-// us, before -> now): 32 queries x 4096 keys x 32 heads 111 -> 21, 1 x 8192 x 32
-// 209 -> 29, 128 x 4096 x 32 111 -> 33, 256 x 256 x 32 19 -> 11, D = 64 2048 x 2048 x 8
-// 48 -> 33, 500 x 500 x 16 of fp32 inputs 25.5 -> 11.
-int attn_parts(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, int sdt) {
+// parts, each 3.5 for the second launch and the partial rows at 6 TB/s (the short
+// kernel's smaller pieces at 3); caches of fp32 inputs pay for the low parts of K.
+// Measured (D = 128 unless stated, bf16 caches, us, before -> now). Short kernel:
+// 32 queries x 4096 keys x 32 heads 111 -> 21, 1 x 8192 x 32 209 -> 29, 128 x 4096
+// x 32 111 -> 33, 256 x 256 x 32 19 -> 11, 500 x 500 x 16 of fp32 inputs, D = 64,
+// 25.5 -> 11. attn_packed_fwd in parts: 4096 x 4096 x 8 123 -> 90, x 4 112 -> 53,
+// 8192 x 8192 x 4 213 -> 152, 2048 x 2048 x 16 64 -> 55, D = 64 6000 x 6000 x 4
+// 120 -> 77, 4096 x 4096 x 8 86 -> 61.
+struct AttnSplit {
+  bool brief;  // attn_packed_short
+  int n;       // key parts
+};
+constexpr AttnSplit kWhole{false, 1};
+
+AttnSplit attn_split(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, int sdt) {
   const int forced = g_force_parts.load(std::memory_order_relaxed);
-  if (forced < 0) return 0;
+  if (forced < 0) return kWhole;
   const int64_t units = ceil_div(Sq, 32) * H * B;
   const int64_t halves = 2 * ceil_div(Skv, BN) + 6;  // at most (four precisions)
   const int64_t most = std::min<int64_t>(ceil_div(halves, ShortCfg<64>::NW), 64);
-  if (units * most >= ((int64_t)1 << 24)) return 0;
-  if (forced > 0) return (int)std::min<int64_t>(forced, most);
+  if (units * most >= ((int64_t)1 << 24)) return kWhole;
+  // attn_packed_fwd: the offsets of a part's rows are 32-bit (see offsets32)
+  const int64_t most_f = offsets32(Skv * H, B, D) ? std::min<int64_t>(ceil_div(halves, 8), 16) : 1;
+  if (forced > 64) return {false, (int)std::min<int64_t>(forced - 64, most_f)};
+  if (forced > 0) return {true, (int)std::min<int64_t>(forced, most)};
   const double lo = sdt == SI_DT_F32 ? 1.45 : 1.0;
-  double best = 0.0;
-  int parts = 0;
+  const double row_us = 8.0 * 32.0 * (double)D * (double)units / 6.0e6;  // per part, both ways
+  AttnSplit best = kWhole;
+  double best_t = 1e30;
+  for (int64_t n = 1; n <= most_f; ++n) {
+    const int64_t blocks = ceil_div(Sq, 256) * H * B * n;
+    const double tile = (blocks > 160 ? 1.25 : 1.0) * (D == 128 ? 1.6 : 1.1) * lo;
+    const double t = (double)ceil_div(blocks, 256) * (9.0 + tile * 0.5 * (double)ceil_div(halves, n)) +
+                     (n > 1 ? 3.5 + row_us * (double)n : 0.0);
+    if (t < best_t) { best_t = t; best = {false, (int)n}; }
+  }
   for (int64_t n = 1; n <= most; ++n) {
-    const double bytes = 8.0 * 32.0 * (double)D * (double)(units * n);
     const double t = (double)ceil_div(units * n, 256) *
                          (6.0 + (D == 128 ? 2.15 : 1.3) * lo * (double)ceil_div(halves, ShortCfg<64>::NW * n)) +
-                     (n > 1 ? 3.5 + bytes / 3.0e6 : 0.0);
-    if (parts == 0 || t < best) { best = t; parts = (int)n; }
+                     (n > 1 ? 3.5 + 2.0 * row_us * (double)n : 0.0);
+    if (t < best_t) { best_t = t; best = {true, (int)n}; }
   }
-  const int64_t blocks = ceil_div(Sq, 256) * H * B;
-  const double tile = (blocks > 128 ? 1.25 : 1.0) * (D == 128 ? 1.6 : 1.1) * lo;
-  const double full = (double)ceil_div(blocks, 256) * (9.0 + tile * 0.5 * (double)halves);
-  return best < full ? parts : 0;
+  return best;
 }
 
 // Workspace of the parts: the partial rows, then their (m, l).
@@ -1554,7 +1609,7 @@ extern "C" void si_tune_attn_parts(int parts) {
 extern "C" size_t si_attn_parts_bytes(int64_t B, int64_t H, int64_t S_q, int64_t D, int64_t S_kv,
                                       int scale_dtype) {
   if (B <= 0 || H <= 0 || S_q <= 0 || S_kv <= 0 || (D != 64 && D != 128)) return 0;
-  return parts_bytes(attn_parts(B, H, S_q, D, S_kv, scale_dtype), B, H, S_q, D);
+  return parts_bytes(attn_split(B, H, S_q, D, S_kv, scale_dtype).n, B, H, S_q, D);
 }
 
 extern "C" void si_tune_attn_offset64(int on) {
@@ -1611,41 +1666,41 @@ int run_attn(const void* q, int q_dtype, int64_t B, int64_t H, int64_t S_q, int6
   const dim3 grid((unsigned)ceil_div(S_q, bmq), (unsigned)H, (unsigned)B);
   const float scale_log2 = sm_scale * 1.4426950408889634f;
   const uint16_t* qp = reinterpret_cast<const uint16_t*>(q);
-  // The wave-per-half-tile kernel where attn_parts expects it to be faster. It
+  // The wave-per-half-tile kernel where attn_split expects it to be faster. It
   // reads 16 bytes of a row per lane and one int4 scale per 8 dims: buckets at
   // other alignments (handed over by a caller) and groups that are no multiple of
   // 8 stay with attn_packed_fwd, as do calls without a workspace for the parts
   // and those that ask for one kernel at every size (split false).
-  int parts = split && group % 8 == 0 ? attn_parts(B, H, S_q, D, S_kv, scale_dtype) : 0;
-  for (int j = 0; j < 16; ++j)
-    if (j % 4 < 2 && (reinterpret_cast<uintptr_t>(bk.p[j]) & 15) != 0) parts = 0;
-  if (parts > 1 && (parts_ws == nullptr || (reinterpret_cast<uintptr_t>(parts_ws) & 15) != 0 ||
-                    parts_ws_bytes < parts_bytes(parts, B, H, S_q, D)))
-    parts = 0;
-  if (parts > 0) {
+  AttnSplit sp = split ? attn_split(B, H, S_q, D, S_kv, scale_dtype) : kWhole;
+  if (sp.brief) {
+    if (group % 8 != 0) sp = kWhole;
+    for (int j = 0; j < 16; ++j)
+      if (j % 4 < 2 && (reinterpret_cast<uintptr_t>(bk.p[j]) & 15) != 0) sp = kWhole;
+  }
+  if (sp.n > 1 && (parts_ws == nullptr || (reinterpret_cast<uintptr_t>(parts_ws) & 15) != 0 ||
+                   parts_ws_bytes < parts_bytes(sp.n, B, H, S_q, D)))
+    sp = kWhole;
+  const bool o32 = offsets32(S_kv * H, B, D);
+  if (sp.brief) {
 #define SI_SHORT_ARGS \
-  q_dtype, scale_dtype, parts, st, qp, B, H, S_q, cap, counts, lists, bk, group, scale_log2, out, out_dtype, os, \
-  offsets32(S_kv * H, B, D), parts_ws
+  q_dtype, scale_dtype, sp.n, st, qp, B, H, S_q, cap, counts, lists, bk, group, scale_log2, out, out_dtype, os, \
+  o32, parts_ws
     if (D == 128) launch_short<128>(SI_SHORT_ARGS);
     else launch_short<64>(SI_SHORT_ARGS);
 #undef SI_SHORT_ARGS
     return check_launch("si_attn_packed_fwd");
   }
+#define SI_FULL_ARGS \
+  scale_dtype, grid, st, qp, B, H, S_q, cap, counts, lists, bk, group, scale_log2, out, out_dtype, os, o32, \
+  sp.n, parts_ws
   if (D == 128) {
-    if (q_dtype == SI_DT_BF16)
-      launch_attn<128, SI_DT_BF16>(scale_dtype, grid, st, qp, B, H, S_q, cap, counts, lists, bk,
-                                   group, scale_log2, out, out_dtype, os, S_kv * H);
-    else
-      launch_attn<128, SI_DT_F16>(scale_dtype, grid, st, qp, B, H, S_q, cap, counts, lists, bk,
-                                  group, scale_log2, out, out_dtype, os, S_kv * H);
+    if (q_dtype == SI_DT_BF16) launch_attn<128, SI_DT_BF16>(SI_FULL_ARGS);
+    else launch_attn<128, SI_DT_F16>(SI_FULL_ARGS);
   } else {
-    if (q_dtype == SI_DT_BF16)
-      launch_attn<64, SI_DT_BF16>(scale_dtype, grid, st, qp, B, H, S_q, cap, counts, lists, bk,
-                                  group, scale_log2, out, out_dtype, os, S_kv * H);
-    else
-      launch_attn<64, SI_DT_F16>(scale_dtype, grid, st, qp, B, H, S_q, cap, counts, lists, bk,
-                                 group, scale_log2, out, out_dtype, os, S_kv * H);
+    if (q_dtype == SI_DT_BF16) launch_attn<64, SI_DT_BF16>(SI_FULL_ARGS);
+    else launch_attn<64, SI_DT_F16>(SI_FULL_ARGS);
   }
+#undef SI_FULL_ARGS
   return check_launch("si_attn_packed_fwd");
 }
 }  // namespace

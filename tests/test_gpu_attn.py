@@ -272,3 +272,50 @@ def test_attention_split_keys_match_oracle(dev, parts, B, H, Sq, S, D, dtype, g,
         assert np.linalg.norm(x - main) <= 2.0 ** -10 * size
     assert torch.equal(token_major.transpose(1, 2), got)
     assert torch.equal(wide, got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [2, 3, 16])
+@pytest.mark.parametrize("B,H,Sq,S,D,dtype,g,probs,evicted", [
+    (1, 2, 300, 700, 128, torch.bfloat16, 16, (1, 1, 1, 1), 0.1),   # ragged second query block
+    (2, 3, 257, 513, 64, torch.float32, 8, (1, 1, 1, 1), 0.2),      # one query past a block
+    (1, 2, 31, 129, 128, torch.float32, 16, (1, 1, 1, 1), 0.1),     # parts that cut between phases
+    (1, 1, 256, 2000, 64, torch.float16, 64, (0, 0, 1, 0), 0.0),    # parts inside one phase
+    (1, 2, 70, 1100, 128, torch.bfloat16, 4, (0, 1, 0, 3), 0.0),    # int4 groups of 4
+    (1, 2, 9, 600, 64, torch.bfloat16, 16, (1, 1, 1, 1), 0.95),     # fewer tiles than parts
+    (1, 2, 40, 400, 128, torch.float16, 16, (1, 1, 1, 1), 1.0),     # every key evicted
+])
+def test_attention_key_parts_match_oracle(dev, parts, B, H, Sq, S, D, dtype, g, probs, evicted):
+    """The 256-query kernel with its tiles split over workgroups, at the edges of
+    its parts, phases and query blocks, in both layouts and against the whole
+    kernel. Bound: the same operands and tiles; the parts round P at other running
+    maxima (2^-11 in each kernel), so as for the wave-per-half-tile kernel."""
+    k, v = kv_inputs(B, H, S, D, dtype, seed=S + D, outlier_frac=0.01)
+    codes = mixed_codes(S, H, seed=S + parts, probs=probs, sink=0 if evicted == 1.0 else 1,
+                        evicted=evicted)
+    if evicted == 1.0:
+        codes[:] = 4
+    cache = _pack(k, v, codes, dev, group_size=g)
+    q = torch.randn(B, H, Sq, D, generator=torch.Generator().manual_seed(S)).to(torch.bfloat16)
+    rk, rv = O.kv_unpack(oracle_pack(k, v, codes, group_size=g))
+    want = O.attention(q.float().numpy().reshape(B * H, Sq, D), rk.reshape(B * H, S, D),
+                       rv.reshape(B * H, S, D)).reshape(B, H, Sq, D).astype(np.float64)
+    lib = _native.load()
+    try:
+        lib.si_tune_attn_parts(-1)
+        main = packed_attention(q.to(dev), cache).cpu().double().numpy()
+        lib.si_tune_attn_parts(64 + parts)
+        got = packed_attention(q.to(dev), cache)
+        token_major = packed_attention(q.to(dev), cache, token_major=True)
+        half = packed_attention(q.to(dev), cache, out_dtype=torch.bfloat16)
+    finally:
+        lib.si_tune_attn_parts(0)
+    x = got.cpu().double().numpy()
+    if evicted == 1.0:
+        assert np.array_equal(x, np.zeros_like(x))
+    else:
+        size = np.linalg.norm(want)
+        assert np.linalg.norm(x - want) <= np.linalg.norm(main - want) + 2.0 ** -11 * size
+        assert np.linalg.norm(x - main) <= 2.0 ** -10 * size
+    assert torch.equal(token_major.transpose(1, 2), got)
+    assert torch.equal(half, got.to(torch.bfloat16))
