@@ -17,12 +17,13 @@ __device__ __forceinline__ float wave_amax(float m) {
 }
 
 // Block-wide |max| for a 256-thread block (4 waves).
+template <int NW = 4>
 __device__ __forceinline__ float block_amax(float m, float* lds) {
   m = wave_amax(m);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = m;
   __syncthreads();
   float r = lds[0];
-  for (int w = 1; w < 4; ++w) r = amax_fold(r, lds[w]);
+  for (int w = 1; w < NW; ++w) r = amax_fold(r, lds[w]);
   __syncthreads();
   return r;
 }
@@ -246,19 +247,19 @@ extern "C" int si_dequant_rows(const int8_t* q, const void* scale, int scale_dty
 }
 
 // Vector form of act_quant_kernel for rows of K % 8 == 0 elements (16-byte
-// aligned rows, K <= 2048 * R, R at most 8; 77 rows of 11008 fp32 values, past the
-// limit of R = 4 before, 23.3 -> 6.3 us): one block per row, the row held in registers
+// aligned rows, K <= 8 * NT * R values; 77 rows of 11008 fp32 values, past the
+// limit of 8192 before, 23.3 -> 4.9 us): one block per row, the row held in registers
 // (R chunks of 8 values per thread), 16-byte loads and 8-byte int8 stores.
 // Same arithmetic: amax, s = max(amax / 127, 1e-8), q = clamp(rint(x / s), +-127)
 // with the IEEE quotient, here Markstein's: q0 = x * RN(1/s), e = x - q0 * s
 // (exact, one fma), RN(q0 + e * RN(1/s)) = RN(x / s) -- no division per value
 // (checked against the division over every bf16 and fp16 row value and 10^8
 // fp32 ones, tests/native/step_quotient_check.c).
-template <int DT, int R>
-__global__ __launch_bounds__(256) void act_quant_vec(const void* __restrict__ x, int64_t M, int K,
+template <int DT, int R, int NT>
+__global__ __launch_bounds__(NT) void act_quant_vec(const void* __restrict__ x, int64_t M, int K,
                                                       int8_t* __restrict__ q,
                                                       float* __restrict__ scale) {
-  __shared__ float lds[4];
+  __shared__ float lds[NT / 64];
   const float eps = 1e-8f;
   const int nch = K / 8;
   for (int64_t m = blockIdx.x; m < M; m += gridDim.x) {
@@ -266,7 +267,7 @@ __global__ __launch_bounds__(256) void act_quant_vec(const void* __restrict__ x,
     float a = 0.0f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int c = (int)threadIdx.x + r * 256;
+      const int c = (int)threadIdx.x + r * NT;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[r][e] = 0.0f;
       if (c < nch) {
@@ -294,14 +295,14 @@ __global__ __launch_bounds__(256) void act_quant_vec(const void* __restrict__ x,
         for (int e = 0; e < 8; ++e) a = amax_fold(a, v[r][e]);
       }
     }
-    a = block_amax(a, lds);
+    a = block_amax<NT / 64>(a, lds);
     float s = a / 127.0f;
     s = s < eps ? eps : s;  // clamp_min(1e-8); NaN passes through like torch
     if (threadIdx.x == 0) scale[m] = s;
     const float rinv = 1.0f / s;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int c = (int)threadIdx.x + r * 256;
+      const int c = (int)threadIdx.x + r * NT;
       if (c >= nch) continue;
       uint32_t b[2] = {0u, 0u};
 #pragma unroll
@@ -316,13 +317,20 @@ __global__ __launch_bounds__(256) void act_quant_vec(const void* __restrict__ x,
   }
 }
 
+// Up to one row per CU a long row is shared by 16 waves instead of 4, whose loads
+// and quotients are a shorter chain: us with 4 and with 16 waves, K = 11008 bf16, M = 1
+// 4.1 and 3.6, 77 4.5 and 4.0, 256 5.4 and 4.4, but 512 (fp32) 7.6 and 8.2, 1024 9.2
+// and 11.3; fp32 at M = 77 4.6 and 3.8. At K <= 8192 both are within 3% to M = 256.
+constexpr int64_t kCuRows = 256;
+
 template <int DT>
 void launch_act_quant_vec(const void* x, int64_t M, int K, int8_t* q, float* scale, unsigned grid,
                           hipStream_t st) {
-  if (K <= 2048) act_quant_vec<DT, 1><<<grid, 256, 0, st>>>(x, M, K, q, scale);
-  else if (K <= 4096) act_quant_vec<DT, 2><<<grid, 256, 0, st>>>(x, M, K, q, scale);
-  else if (K <= 8192) act_quant_vec<DT, 4><<<grid, 256, 0, st>>>(x, M, K, q, scale);
-  else act_quant_vec<DT, 8><<<grid, 256, 0, st>>>(x, M, K, q, scale);
+  if (K <= 2048) act_quant_vec<DT, 1, 256><<<grid, 256, 0, st>>>(x, M, K, q, scale);
+  else if (K <= 4096) act_quant_vec<DT, 2, 256><<<grid, 256, 0, st>>>(x, M, K, q, scale);
+  else if (K <= 8192) act_quant_vec<DT, 4, 256><<<grid, 256, 0, st>>>(x, M, K, q, scale);
+  else if (M <= kCuRows) act_quant_vec<DT, 2, 1024><<<grid, 1024, 0, st>>>(x, M, K, q, scale);
+  else act_quant_vec<DT, 8, 256><<<grid, 256, 0, st>>>(x, M, K, q, scale);
 }
 
 extern "C" int si_act_quant_i8(const void* x, int dtype, int64_t M, int64_t K, int8_t* q,

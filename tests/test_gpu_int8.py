@@ -454,3 +454,26 @@ def test_wide_rows_and_split_sums_match_oracle(dev, dtype, M, K, N):
     want, _, _, _ = O.int8_linear_forward(to_np(x), DT[dtype], w.t().contiguous().numpy(),
                                           sw.numpy(), bs.numpy())
     np.testing.assert_array_equal(to_np(y), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K", [(1, 8200), (256, 8200), (257, 8200), (256, 11008), (257, 11008),
+                                 (2, 16384), (258, 16384)])
+def test_long_row_quantization_up_to_a_row_per_cu(dev, dtype, M, K):
+    """Rows of 8193..16384 values on either side of the 256 rows up to which 16
+    waves share one: the int8 values and scales equal the reference's fp32 ops
+    (amax / 127, clamp, x / s, round), a row of zeros included."""
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)).to(dtype)
+    x[:, -1] *= 9.0       # the last value of a row decides its scale
+    x[M // 2] = 0.0
+    q = torch.empty(M, K, dtype=torch.int8, device=dev)
+    s = torch.empty(M, dtype=torch.float32, device=dev)
+    xd = x.to(dev)
+    _native.call("si_act_quant_i8", xd.data_ptr(), _native.dtype_code(dtype), M, K, q.data_ptr(),
+                 s.data_ptr(), _native.stream(dev))
+    f = x.float()
+    want_s = (f.abs().amax(dim=1) / 127.0).clamp_min(1e-8)
+    want_q = (f / want_s[:, None]).round().clamp(-127, 127).to(torch.int8)
+    assert torch.equal(s.cpu(), want_s)
+    assert torch.equal(q.cpu(), want_q)
