@@ -201,6 +201,44 @@ def test_cpu_tensors_fail_loudly():
         INT8Linear.from_linear(nn.Linear(8, 8))
 
 
+def test_cpu_caches_stop_before_any_launch(monkeypatch):
+    """A cache whose tensors are in host memory (as after ``torch.load(...,
+    map_location="cpu")``) and a hand-over of CPU int4 rows raise ValueError, as
+    torch.cuda.current_stream does for such a device, and launch nothing: every
+    call and handle lookup is stubbed, as on a machine with a GPU."""
+    from shadowinfer_amd.shadowkv.packed_kv_cache import _pack_rows
+    from shadowinfer_amd.shadowkv.precision_plan import DeviceGrouping
+    launched = []
+    monkeypatch.setattr(_native, "call", lambda name, *args: launched.append(name))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    S, H, D = 6, 2, 64
+
+    def cache():
+        c = PackedKVCache(1, H, S, D)
+        c._grouping = DeviceGrouping(torch.full((S * H,), 1, dtype=torch.int8),
+                                     torch.arange(S * H, dtype=torch.int32), [0, S * H, 0, 0, 0],
+                                     [torch.empty(n, dtype=torch.long) for n in (0, S * H, 0, 0)])
+        c._group_size, c._scale_dtype = 16, torch.float32
+        c._buckets = c._alloc_buckets(c._grouping.counts, torch.device("cpu"), torch.float32)
+        return c
+
+    mask = torch.ones(S, H, dtype=torch.bool)
+    unbuilt = DeviceGrouping(cache()._grouping.code, cache()._grouping.slot, [0, S * H, 0, 0, 0])
+    for use in (lambda: cache().unpack(),
+                lambda: cache().evict(mask),
+                lambda: cache().evict({(0, 0)}),
+                lambda: cache().apply_reuse_mask(cache(), mask),
+                lambda: cache().attention_lists(),
+                lambda: unbuilt.flat_lists(S, H),
+                lambda: _pack_rows(torch.zeros(3, 64, dtype=torch.int8)),
+                lambda: _native.stream(torch.device("cpu"))):
+        with pytest.raises(ValueError, match="cuda device"):
+            use()
+    assert launched == []
+    assert _native.stream(torch.device("cuda")) == 0 == _native.stream(torch.device("cuda", 0))
+
+
 def test_rope_pack_rejects_bad_tables_before_any_launch():
     """pack_projection reads cos/sin [S, D] in qkv's dtype for every token: a
     short table or one of another dtype is a ValueError (a short table would be
