@@ -376,11 +376,12 @@ __global__ __launch_bounds__(256) void swiglu_quant(const void* __restrict__ gu,
 // One block per row. A row of up to 256 * 8 * R values stays in registers
 // (row_argmax_conf_regs): one read of the logits instead of three passes of
 // which the later two came from L2. The kernel is bound by its VALU work on
-// every logit, so the exponential is exp2 of a two-term product (row_exp: 4
-// instructions for expf's 12) and no pass looks for NaN or infinities: a row
-// that holds one (or only -inf) has a NaN sum. 2048 rows of 32000 bf16 logits
-// 70 -> 37 us (131 MB: 26 us at the copy rate), of 32001 fp16 162 -> 38, 1024 rows
-// of 32000 fp32 58 -> 33, 8 rows of 32000 bf16 20 -> 11.
+// every logit, so no pass looks for NaN or infinities (a row that holds one, or
+// only -inf, has a NaN sum) and the sum takes expf's bits from row_exp: 10
+// instructions for 15, 2048 rows of 32000 bf16 logits 38 us against 43 with expf
+// itself (33 with exp2 of a rounded d * log2(e), up to 45 ulp off: not kept).
+// 2048 rows of 32000 bf16 65 -> 38 us (131 MB: 26 us at the copy rate), of 32001
+// fp16 138 -> 40, of 32000 fp32 113 -> 59, 8 rows of 32000 bf16 20 -> 12.
 // ---------------------------------------------------------------------------
 template <int DT, bool VEC, typename F>
 __device__ __forceinline__ void for_row(const void* __restrict__ logits, int64_t m, int64_t V,
@@ -397,10 +398,20 @@ __device__ __forceinline__ void for_row(const void* __restrict__ logits, int64_t
   }
 }
 
-// exp(d) for d <= 0, within 2 ulp plus |d| 2^-24: exp2 of d * log2(e) with the
-// constant in two terms (a single one would shift every term the same way).
+// exp(d) for d <= 0 (NaN stays NaN): d * log2(e) as an exact product h + l, the
+// nearest integer e of h, 2^(h - e + l) on v_exp_f32 and e added to its exponent.
+// Of all floats from -87 to 0, all but 16 give expf's bits, and the largest error is
+// expf's (0.857 ulp; mean 0.257 in both). Below -87 it gives exp(-87) = 1.6e-38
+// where expf falls to 0: the sum it goes into holds expf(0) = 1.
 __device__ __forceinline__ float row_exp(float d) {
-  return __builtin_amdgcn_exp2f(__builtin_fmaf(d, 1.44269502f, d * 1.92596303e-8f));
+  constexpr float kHi = 1.44269502f, kLo = 1.92596303e-8f;  // log2(e)
+  constexpr float kRound = 12582912.0f;                     // 1.5 * 2^23
+  d = __builtin_elementwise_maximum(d, -87.0f);
+  const float h = d * kHi;
+  const float l = __builtin_fmaf(d, kLo, __builtin_fmaf(d, kHi, -h));
+  const float t = h + kRound, e = t - kRound;
+  const float r = __builtin_amdgcn_exp2f((h - e) + l);
+  return __uint_as_float(__float_as_uint(r) + (__float_as_uint(t) << 23));
 }
 
 // The row's result from thread-wise first candidates (INT64_MAX: none).

@@ -825,6 +825,36 @@ def test_argmax_conf_row_lengths(dev, dtype, M, V):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("V", [2048, 32000, 32776, 40000])  # registers; from 32776 on three passes
+def test_confidence_sum_adds_the_library_exponential(dev, V):
+    """One peak over V - 1 equal logits, where an error of the exponential is the
+    same in every term: the fp32 confidence is 1 / the sum of the library's expf
+    values (torch.exp on the device), added in the kernel's order (eight values of
+    256 threads in turn, a butterfly over 64 lanes, then pairs of waves). Exact:
+    the kernel's exponential has expf's bits at all of these arguments."""
+    from shadowinfer_amd.execution import argmax_confidence
+    d = torch.cat([torch.linspace(-86.9, -0.07, 128), torch.linspace(-13.0, -5.0, 512)])
+    x = d[:, None].repeat(1, V)
+    x[:, 0] = 0.0
+    x = x.to(dev)
+    _, conf = argmax_confidence(x)
+    units = -(-V // 2048)
+    term = torch.zeros(len(d), units * 2048, device=dev)
+    term[:, :V] = torch.exp(x)
+    term = term.view(len(d), units, 256, 8)
+    s = torch.zeros(len(d), 256, device=dev)
+    for u in range(units):
+        for e in range(8):
+            s = s + term[:, u, :, e]
+    s = s.view(len(d), 4, 64)
+    for off in (32, 16, 8, 4, 2, 1):
+        s = s + s[:, :, torch.arange(64, device=dev) ^ off]
+    s = s[:, :, 0]
+    want = 1.0 / ((s[:, 0] + s[:, 1]) + (s[:, 2] + s[:, 3]))
+    assert torch.equal(conf, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W", [1, 63, 1024, 1025, 3000])
 def test_schedule_rows_nan_ties_and_signs(dev, W):
     """The unmasking rule with NaN confidences (largest for the fallback, NaN kept
