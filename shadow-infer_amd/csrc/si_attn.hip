@@ -1215,11 +1215,12 @@ __global__ __launch_bounds__(512) void attn_packed_short(
     // fp32 rows are read in two steps (K, then V): 32 bytes of each of K and V
     // per lane and row would not fit the registers.
     constexpr bool BOTH = P != SI_PREC_FP32;
+    constexpr bool LATE_V = P == SI_PREC_FP32 || (INT && KLO);  // V to LDS after the scores
     uint32_t rk[RPL][W], rv[BOTH ? RPL : 1][W], skb[RPL], svb[RPL], us[RPL];
     auto load_rows = [&](int uu) __attribute__((always_inline)) {
       const int nv = n_end - uu * HN;
       // Keys past the phase's last read row 0 of the (non-empty) bucket: their
-      // list entries are not written; their scores are masked.
+      // list entries are not written; their scores are masked, their V cleared.
 #pragma unroll
       for (int i = 0; i < RPL; ++i) {
         us[i] = (uint32_t)(row0 + i < nv ? sl[i] : 0);
@@ -1291,6 +1292,15 @@ __global__ __launch_bounds__(512) void attn_packed_short(
     auto put_k = [&](int r, uint4 w) __attribute__((always_inline)) { *reinterpret_cast<uint4*>(&Kt[r][d0]) = w; };
     auto put_l = [&](int r, uint4 w) __attribute__((always_inline)) { *reinterpret_cast<uint4*>(&Kl[r][d0]) = w; };
     auto put_v = [&](int r, uint4 w) __attribute__((always_inline)) { *reinterpret_cast<uint4*>(&Vt[r][d0]) = w; };
+    // V of the keys past the phase's last (a wave-uniform branch, in its last half
+    // tile): what they read is another head's row, and one of its values may be
+    // infinite in fp16, which P = 0 does not cancel.
+    auto clear_v = [&](int nv) __attribute__((always_inline)) {
+      if (nv == HN) return;
+#pragma unroll
+      for (int i = 0; i < RPL; ++i)
+        if (row0 + i >= nv) put_v(row0 + i, make_uint4(0u, 0u, 0u, 0u));
+    };
 
     load_rows(u);
     while (true) {
@@ -1331,6 +1341,7 @@ __global__ __launch_bounds__(512) void attn_packed_short(
         decode(rk, skb, put_k);
         decode(rv, svb, put_v);
       }
+      if constexpr (!LATE_V) clear_v(nv);
       if constexpr (P == SI_PREC_FP32) {  // V, into the registers of K
 #pragma unroll
         for (int i = 0; i < RPL; ++i) {
@@ -1341,7 +1352,6 @@ __global__ __launch_bounds__(512) void attn_packed_short(
       }
       wave_lds_order();
       // Rows of the next half tile, unless this one's V is still in registers.
-      constexpr bool LATE_V = P == SI_PREC_FP32 || (INT && KLO);
       if constexpr (!LATE_V)
         if (nx < he) load_rows(nx);
       v16f sacc[1];
@@ -1362,6 +1372,7 @@ __global__ __launch_bounds__(512) void attn_packed_short(
         } else {
           decode(rv, svb, put_v);
         }
+        clear_v(nv);
         wave_lds_order();
         if (nx < he) load_rows(nx);
       }

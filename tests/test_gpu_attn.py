@@ -319,3 +319,35 @@ def test_attention_key_parts_match_oracle(dev, parts, B, H, Sq, S, D, dtype, g, 
         assert np.linalg.norm(x - main) <= 2.0 ** -10 * size
     assert torch.equal(token_major.transpose(1, 2), got)
     assert torch.equal(half, got.to(torch.bfloat16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,code,parts", [
+    (torch.float32, 0, -1), (torch.float32, 0, 1), (torch.float32, 0, 3), (torch.float32, 0, 64 + 2),
+    (torch.bfloat16, 0, 2), (torch.bfloat16, 1, 1), (torch.bfloat16, 2, 2), (torch.bfloat16, 3, 1),
+    (torch.float32, 2, 1), (torch.float32, 3, 2)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_attention_values_past_fp16_stay_in_their_head(dev, D, dtype, code, parts):
+    """Head 0's first value row is 1e5, infinite as an fp16 operand; the other
+    heads' keys end inside a tile, where the rows past the last key are read from
+    the bucket's first row: head 0's. Those heads match the oracle (bounds of
+    this file: 1e-3; their own operands are of ordinary size)."""
+    B, H, Sq, S = 1, 3, 40, 101
+    k, v = kv_inputs(B, H, S, D, dtype, seed=D + code)
+    v[:, 0, 0] = 1e5
+    codes = np.full((S, H), code, np.int8)
+    codes[50:, 1] = (code + 1) % 4
+    codes[37:, 2] = 4
+    cache = _pack(k, v, codes, dev)
+    q = torch.randn(B, H, Sq, D, generator=torch.Generator().manual_seed(D)).to(torch.bfloat16)
+    lib = _native.load()
+    lib.si_tune_attn_parts(parts)
+    try:
+        out = packed_attention(q.to(dev), cache).cpu().numpy()[:, 1:]
+    finally:
+        lib.si_tune_attn_parts(0)
+    rk, rv = (x[:, 1:] for x in O.kv_unpack(oracle_pack(k, v, codes)))
+    ref = O.attention(np.ascontiguousarray(q.float().numpy()[:, 1:]).reshape(2, Sq, D),
+                      np.ascontiguousarray(rk).reshape(2, S, D),
+                      np.ascontiguousarray(rv).reshape(2, S, D)).reshape(B, 2, Sq, D)
+    assert _rel_l2(out, ref) <= TOL
