@@ -1529,20 +1529,36 @@ std::atomic<int> g_force_parts{0};
 // The rule compares time estimates (us), fitted on S_kv = 100..8192, H = 4..32:
 // attn_packed_fwd takes 9 + 1.6 per 64-key tile and round of 256 blocks (D = 64:
 // 1.1; a quarter more where its blocks fill over 160 CUs, as the clock then drops),
-// the short kernel 6 + 2.15 per half tile and wave (D = 64: 1.3) and, with n > 1
-// parts, each 3.5 for the second launch and the partial rows at 6 TB/s (the short
-// kernel's smaller pieces at 3); caches of fp32 inputs pay for the low parts of K.
+// the short kernel 6 + 2.15 per half tile and wave (D = 64: 1.3; 3.55 with the low
+// parts of K at D = 128) and, with n > 1 parts, each 3.5 for the second launch and
+// the partial rows at 6 TB/s (the short kernel's smaller pieces at 3); caches of
+// fp32 inputs pay for the low parts of K.
 // Measured (D = 128 unless stated, bf16 caches, us, before -> now). Short kernel:
 // 32 queries x 4096 keys x 32 heads 111 -> 21, 1 x 8192 x 32 209 -> 29, 128 x 4096
 // x 32 111 -> 33, 256 x 256 x 32 19 -> 11, 500 x 500 x 16 of fp32 inputs, D = 64,
 // 25.5 -> 11. attn_packed_fwd in parts: 4096 x 4096 x 8 123 -> 90, x 4 112 -> 53,
 // 8192 x 8192 x 4 213 -> 152, 2048 x 2048 x 16 64 -> 55, D = 64 6000 x 6000 x 4
 // 120 -> 77, 4096 x 4096 x 8 86 -> 61.
+//
+// Long calls run at a lower clock the fuller the chip is, so there an estimate
+// must promise 10%: of those that promised 1-6%, most lost up to 9% (us whole and
+// split: 8 heads, S = S_q = 5384, D = 64, fp32 170 and 186, 32 x 7168 885 and 913, 12
+// x 3584 102 and 110), where under 60 us they gained 2-26%. The partial rows have to
+// fit kPartsMax: they grow with every query (32 x 7168 239 MB, 12 heads at 262400
+// keys 4.9 GB) beside an output that fits without them, and the largest split that
+// gained in the range above takes 134 MB (12 x 7168: 415 -> 363).
 struct AttnSplit {
   bool brief;  // attn_packed_short
   int n;       // key parts
 };
 constexpr AttnSplit kWhole{false, 1};
+constexpr size_t kPartsMax = (size_t)128 << 20;
+
+// Workspace of the parts: the partial rows, then their (m, l).
+size_t parts_bytes(int64_t parts, int64_t B, int64_t H, int64_t Sq, int64_t D) {
+  if (parts <= 1) return 0;
+  return (size_t)(ceil_div(Sq, 32) * H * B) * (size_t)parts * 32 * (size_t)(D + 2) * sizeof(float);
+}
 
 AttnSplit attn_split(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, int sdt) {
   const int forced = g_force_parts.load(std::memory_order_relaxed);
@@ -1559,26 +1575,22 @@ AttnSplit attn_split(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, i
   const double row_us = 8.0 * 32.0 * (double)D * (double)units / 6.0e6;  // per part, both ways
   AttnSplit best = kWhole;
   double best_t = 1e30;
-  for (int64_t n = 1; n <= most_f; ++n) {
+  for (int64_t n = 1; n <= most_f && parts_bytes(n, B, H, Sq, D) <= kPartsMax; ++n) {
     const int64_t blocks = ceil_div(Sq, 256) * H * B * n;
     const double tile = (blocks > 160 ? 1.25 : 1.0) * (D == 128 ? 1.6 : 1.1) * lo;
     const double t = (double)ceil_div(blocks, 256) * (9.0 + tile * 0.5 * (double)ceil_div(halves, n)) +
                      (n > 1 ? 3.5 + row_us * (double)n : 0.0);
-    if (t < best_t) { best_t = t; best = {false, (int)n}; }
+    if (n == 1) best_t = t < 60.0 ? t : t / 1.1;
+    else if (t < best_t) { best_t = t; best = {false, (int)n}; }
   }
-  for (int64_t n = 1; n <= most; ++n) {
+  const double half_us = D == 64 ? 1.3 * lo : sdt == SI_DT_F32 ? 3.55 : 2.15;
+  for (int64_t n = 1; n <= most && parts_bytes(n, B, H, Sq, D) <= kPartsMax; ++n) {
     const double t = (double)ceil_div(units * n, 256) *
-                         (6.0 + (D == 128 ? 2.15 : 1.3) * lo * (double)ceil_div(halves, ShortCfg<64>::NW * n)) +
+                         (6.0 + half_us * (double)ceil_div(halves, ShortCfg<64>::NW * n)) +
                      (n > 1 ? 3.5 + 2.0 * row_us * (double)n : 0.0);
     if (t < best_t) { best_t = t; best = {true, (int)n}; }
   }
   return best;
-}
-
-// Workspace of the parts: the partial rows, then their (m, l).
-size_t parts_bytes(int parts, int64_t B, int64_t H, int64_t Sq, int64_t D) {
-  if (parts <= 1) return 0;
-  return (size_t)(ceil_div(Sq, 32) * H * B) * (size_t)parts * 32 * (size_t)(D + 2) * sizeof(float);
 }
 
 template <int D>

@@ -29,10 +29,11 @@ def packed_attention(q: torch.Tensor, cache: PackedKVCache, sm_scale: Optional[f
     by the kernel: the ``attn.transpose(1, 2)`` layout an output projection
     reads (models/diffusion_llama.py:390-391).
 
-    Calls with few queries or heads have their keys split over workgroups, and
-    then round P at other running maxima (the error against float64 is the
-    same). ``split_keys=False`` keeps one kernel, and so the same bits for a
-    query row, at every ``S_q`` and ``H``."""
+    Calls whose 256-query blocks leave CUs idle (few queries, few heads, a partly
+    filled last round) have their keys split over workgroups, through at most
+    128 MiB of partial results, and then round P at other running maxima (the
+    error against float64 is the same). ``split_keys=False`` keeps one kernel, and
+    so the same bits for a query row, at every ``S_q`` and ``H``."""
     if q.dim() != 4:
         raise ValueError(f"q must be [batch, heads, seq, dim], got {tuple(q.shape)}")
     B, H, Sq, D = q.shape

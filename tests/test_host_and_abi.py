@@ -127,6 +127,30 @@ def test_workspace_queries():
     assert _native.size_query("si_int8_linear_workspace_bytes", 16, 4096, 11008) >= 16 * 4096
 
 
+def test_attention_parts_workspace_is_bounded():
+    """A split's partial rows stay within 128 MiB at any size (the output of such a
+    call fitted without them), and calls where a split gains nothing (32 heads,
+    7168 x 7168) stay whole. Few queries or heads are split."""
+    def parts(B, H, Sq, D, S, dt):
+        return _native.size_query("si_attn_parts_bytes", B, H, Sq, D, S, dt)
+
+    for B in (1, 2, 16):
+        for H in (1, 4, 12, 32, 128):
+            for S in (1, 100, 700, 3000, 6000, 7168, 8192, 70000, 262400):
+                for Sq in {1, 32, 256, S}:
+                    for D in (64, 128):
+                        for dt in (0, 2):
+                            got = parts(B, H, Sq, D, S, dt)
+                            unit = -(-Sq // 32) * H * B * 32 * (D + 2) * 4
+                            assert got <= 128 << 20 and got % unit == 0 and got != unit
+    for D in (64, 128):
+        assert parts(1, 32, 7168, D, 7168, 2) == 0
+        assert parts(1, 32, 3000, D, 3000, 2) == 0
+        assert parts(1, 32, 32, D, 4096, 2) > 0
+        assert parts(1, 4, 8192, D, 8192, 2) > 0
+        assert parts(1, 12, 6000, D, 6000, 2) > 0
+
+
 # ------------------------------------------------------- codes and plans
 def test_map_to_codes_and_back_match_reference_semantics():
     pm = {0: {0: "fp32", 2: "evicted"}, 1: {1: "INT8"}, 2: {0: "int4", 1: "fp16", 2: "fp32"},
