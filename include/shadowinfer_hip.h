@@ -309,10 +309,11 @@ int si_attn_packed_fwd_built(const void* q, int q_dtype, int64_t B, int64_t H, i
  * leave CUs idle (few queries, few heads, or a last round of 256 blocks that is
  * partly filled): their keys are then split over workgroups, whose partial
  * results pass through the workspace. si_attn_parts_bytes is what a call of that
- * shape takes (0 for most, at most 128 MiB); with a smaller or NULL workspace
- * (16-byte aligned) the keys are not split. A split
+ * shape takes (0 for most, at most 128 MiB); with less (16-byte aligned) the keys
+ * are split in fewer parts, with NULL they are not. A split
  * call rounds the probabilities at other running maxima: split == 0 keeps one
- * kernel, so the same bits for a query row, at every size. */
+ * kernel, so the same bits for a query row, at every size. (The entry points
+ * above choose between two kernels by shape, as split != 0 with NULL does.) */
 size_t si_attn_parts_bytes(int64_t B, int64_t H, int64_t S_q, int64_t D, int64_t S_kv,
                            int scale_dtype);
 int si_attn_packed_fwd_parts(const void* q, int q_dtype, int64_t B, int64_t H, int64_t S_q,

@@ -1560,7 +1560,10 @@ size_t parts_bytes(int64_t parts, int64_t B, int64_t H, int64_t Sq, int64_t D) {
   return (size_t)(ceil_div(Sq, 32) * H * B) * (size_t)parts * 32 * (size_t)(D + 2) * sizeof(float);
 }
 
-AttnSplit attn_split(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, int sdt) {
+// The fastest that the call allows: attn_packed_short only with brief_ok, parts
+// whose rows fit ws_max bytes.
+AttnSplit attn_split(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, int sdt, bool brief_ok,
+                     size_t ws_max) {
   const int forced = g_force_parts.load(std::memory_order_relaxed);
   if (forced < 0) return kWhole;
   const int64_t units = ceil_div(Sq, 32) * H * B;
@@ -1569,13 +1572,17 @@ AttnSplit attn_split(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, i
   if (units * most >= ((int64_t)1 << 24)) return kWhole;
   // attn_packed_fwd: the offsets of a part's rows are 32-bit (see offsets32)
   const int64_t most_f = offsets32(Skv * H, B, D) ? std::min<int64_t>(ceil_div(halves, 8), 16) : 1;
-  if (forced > 64) return {false, (int)std::min<int64_t>(forced - 64, most_f)};
-  if (forced > 0) return {true, (int)std::min<int64_t>(forced, most)};
+  if (forced > 0) {
+    const AttnSplit f = forced > 64 ? AttnSplit{false, (int)std::min<int64_t>(forced - 64, most_f)}
+                                    : AttnSplit{true, (int)std::min<int64_t>(forced, most)};
+    return (f.brief && !brief_ok) || parts_bytes(f.n, B, H, Sq, D) > ws_max ? kWhole : f;
+  }
+  const size_t fits = std::min(ws_max, kPartsMax);
   const double lo = sdt == SI_DT_F32 ? 1.45 : 1.0;
   const double row_us = 8.0 * 32.0 * (double)D * (double)units / 6.0e6;  // per part, both ways
   AttnSplit best = kWhole;
   double best_t = 1e30;
-  for (int64_t n = 1; n <= most_f && parts_bytes(n, B, H, Sq, D) <= kPartsMax; ++n) {
+  for (int64_t n = 1; n <= most_f && parts_bytes(n, B, H, Sq, D) <= fits; ++n) {
     const int64_t blocks = ceil_div(Sq, 256) * H * B * n;
     const double tile = (blocks > 160 ? 1.25 : 1.0) * (D == 128 ? 1.6 : 1.1) * lo;
     const double t = (double)ceil_div(blocks, 256) * (9.0 + tile * 0.5 * (double)ceil_div(halves, n)) +
@@ -1584,7 +1591,7 @@ AttnSplit attn_split(int64_t B, int64_t H, int64_t Sq, int64_t D, int64_t Skv, i
     else if (t < best_t) { best_t = t; best = {false, (int)n}; }
   }
   const double half_us = D == 64 ? 1.3 * lo : sdt == SI_DT_F32 ? 3.55 : 2.15;
-  for (int64_t n = 1; n <= most && parts_bytes(n, B, H, Sq, D) <= kPartsMax; ++n) {
+  for (int64_t n = 1; brief_ok && n <= most && parts_bytes(n, B, H, Sq, D) <= fits; ++n) {
     const double t = (double)ceil_div(units * n, 256) *
                          (6.0 + half_us * (double)ceil_div(halves, ShortCfg<64>::NW * n)) +
                      (n > 1 ? 3.5 + 2.0 * row_us * (double)n : 0.0);
@@ -1632,7 +1639,7 @@ extern "C" void si_tune_attn_parts(int parts) {
 extern "C" size_t si_attn_parts_bytes(int64_t B, int64_t H, int64_t S_q, int64_t D, int64_t S_kv,
                                       int scale_dtype) {
   if (B <= 0 || H <= 0 || S_q <= 0 || S_kv <= 0 || (D != 64 && D != 128)) return 0;
-  return parts_bytes(attn_split(B, H, S_q, D, S_kv, scale_dtype).n, B, H, S_q, D);
+  return parts_bytes(attn_split(B, H, S_q, D, S_kv, scale_dtype, true, SIZE_MAX).n, B, H, S_q, D);
 }
 
 extern "C" void si_tune_attn_offset64(int on) {
@@ -1689,20 +1696,22 @@ int run_attn(const void* q, int q_dtype, int64_t B, int64_t H, int64_t S_q, int6
   const dim3 grid((unsigned)ceil_div(S_q, bmq), (unsigned)H, (unsigned)B);
   const float scale_log2 = sm_scale * 1.4426950408889634f;
   const uint16_t* qp = reinterpret_cast<const uint16_t*>(q);
-  // The wave-per-half-tile kernel where attn_split expects it to be faster. It
-  // reads 16 bytes of a row per lane and one int4 scale per 8 dims: buckets at
-  // other alignments (handed over by a caller) and groups that are no multiple of
-  // 8 stay with attn_packed_fwd, as do calls without a workspace for the parts
-  // and those that ask for one kernel at every size (split false).
-  AttnSplit sp = split ? attn_split(B, H, S_q, D, S_kv, scale_dtype) : kWhole;
-  if (sp.brief) {
-    if (group % 8 != 0) sp = kWhole;
+  // The wave-per-half-tile kernel reads 16 bytes of a row per lane and one int4
+  // scale per 8 dims: buckets at other alignments (handed over by a caller) and
+  // groups that are no multiple of 8 leave attn_packed_fwd, whose keys are split
+  // where that pays in the workspace at hand; calls without one take the better of
+  // the two kernels in one part, and those that ask for one kernel at every size
+  // (split false) attn_packed_fwd whole. 32 queries x 4096 keys x 32 heads, D = 64,
+  // groups of 4: 83 us whole, 31 in parts; D = 128 without a workspace 110 us, 42 on
+  // attn_packed_short.
+  AttnSplit sp = kWhole;
+  if (split) {
+    bool brief_ok = group % 8 == 0;
     for (int j = 0; j < 16; ++j)
-      if (j % 4 < 2 && (reinterpret_cast<uintptr_t>(bk.p[j]) & 15) != 0) sp = kWhole;
+      if (j % 4 < 2 && (reinterpret_cast<uintptr_t>(bk.p[j]) & 15) != 0) brief_ok = false;
+    const bool ws = parts_ws != nullptr && (reinterpret_cast<uintptr_t>(parts_ws) & 15) == 0;
+    sp = attn_split(B, H, S_q, D, S_kv, scale_dtype, brief_ok, ws ? parts_ws_bytes : 0);
   }
-  if (sp.n > 1 && (parts_ws == nullptr || (reinterpret_cast<uintptr_t>(parts_ws) & 15) != 0 ||
-                   parts_ws_bytes < parts_bytes(sp.n, B, H, S_q, D)))
-    sp = kWhole;
   const bool o32 = offsets32(S_kv * H, B, D);
   if (sp.brief) {
 #define SI_SHORT_ARGS \

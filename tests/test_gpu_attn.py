@@ -351,3 +351,47 @@ def test_attention_values_past_fp16_stay_in_their_head(dev, D, dtype, code, part
                       np.ascontiguousarray(rk).reshape(2, S, D),
                       np.ascontiguousarray(rv).reshape(2, S, D)).reshape(B, 2, Sq, D)
     assert _rel_l2(out, ref) <= TOL
+
+
+@pytest.mark.gpu
+def test_attention_takes_the_best_split_that_the_call_allows(dev):
+    """Where the fastest split cannot be used, the best remaining one is, not the
+    whole kernel: caches with int4 groups of 4 (no wave-per-half-tile kernel) split
+    the 256-query kernel in the workspace they were given, and the entry points
+    without a workspace take the wave-per-half-tile kernel in one part (equal bits
+    with either forced). A workspace too small for any part leaves one part."""
+    lib = _native.load()
+    B, H, Sq, S, D = 1, 8, 32, 2048, 64
+
+    def forced(cache, q, parts):
+        lib.si_tune_attn_parts(parts)
+        try:
+            return packed_attention(q, cache)
+        finally:
+            lib.si_tune_attn_parts(0)
+
+    k, v = kv_inputs(B, H, S, D, torch.bfloat16, seed=3)
+    codes = mixed_codes(S, H, seed=3, probs=(0, 1, 2, 1), sink=4)
+    q = torch.randn(B, H, Sq, D, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(dev)
+    narrow = _pack(k, v, codes, dev, group_size=4)
+    got, whole = packed_attention(q, narrow), forced(narrow, q, -1)
+    assert not torch.equal(got, whole)
+    assert any(torch.equal(got, forced(narrow, q, 64 + n)) for n in range(2, 17))
+    cache = _pack(k, v, codes, dev)
+    code, slot, table, sdt, group = cache.device_state()
+    ws_bytes = _native.size_query("si_attn_workspace_bytes", H, S)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    out = torch.empty(B, H, Sq, D, dtype=torch.float32, device=dev)
+    _native.call("si_attn_packed_fwd", q.data_ptr(), _native.dtype_code(q.dtype), B, H, Sq, D,
+                 code.data_ptr(), slot.data_ptr(), table, sdt, S, group, float(1 / D ** 0.5),
+                 out.data_ptr(), _native.dtype_code(torch.float32), ws.data_ptr(), ws_bytes,
+                 _native.stream(dev))
+    one = forced(cache, q, 1)
+    assert torch.equal(out, one) and not torch.equal(out, forced(cache, q, -1))
+    lists = cache.attention_lists()
+    small = torch.empty(64, dtype=torch.uint8, device=dev)
+    _native.call("si_attn_packed_fwd_parts", q.data_ptr(), _native.dtype_code(q.dtype), B, H, Sq, D,
+                 lists.data_ptr(), lists.numel(), table, sdt, S, group, float(1 / D ** 0.5),
+                 out.data_ptr(), _native.dtype_code(torch.float32), 0, 1, small.data_ptr(), 64,
+                 _native.stream(dev))
+    assert torch.equal(out, one)
