@@ -23,14 +23,20 @@
 // once, and at most kAdmBlocks blocks add to the same few counters: 10 launches
 // for 30. (Handing over to the last block of a pass instead took as long as the
 // 30 launches: its device-scope fences write back and drop the L2s, 20 us each.)
-// The solver with eviction at 8192 x 32: 195 -> 55 us of kernels.
+// The solver with eviction at 8192 x 32: 179 -> 52 us of kernels.
 #include "si_common.h"
 
 namespace si {
 namespace {
 
 constexpr int ADM_THREADS = 1024;
-constexpr int64_t kAdmBlocks = 64;
+// A block per CU. The solver with eviction in us, by the most blocks that add to
+// the counters (and with one launch per step and 2048 small blocks, before):
+//   entries   64   128   256   512  before
+//     1.0 M   82    70    71    72     295
+//     4.2 M  250   154   121   133     341
+//      17 M  951   540   344   299     602
+constexpr int64_t kAdmBlocks = 256;
 constexpr int TIE_CHUNK = 2 * ADM_THREADS;  // entries per block of the tie scan
 constexpr int BINS = 2048;                  // of a digit's histogram
 constexpr int MODE_DOWN = 0;     // ladder downgrade (fp32 -> fp16 -> int8 -> int4)
