@@ -1112,7 +1112,7 @@ __global__ __launch_bounds__(256) void kv_unpack_sorted(const int8_t* __restrict
 // 0..3 (evicted or absent). blk_end[p]: first block after precision p's.
 
 // DC: the head dim where it is a compile-time constant, else 0 (any multiple
-// of 4 up to 4 * NT, the block's last NT % (D / 4) threads idle).
+// of 16 up to 192, the block's last NT % (D / 4) threads idle).
 template <int DC, int SDT, int U, int P, int NT>
 __device__ __forceinline__ void unpack_bucket_rows(const UnpackLists& L, const Buckets& bk,
                                                    int64_t lb, int B, int64_t HS, int Dr, int g,
@@ -2537,9 +2537,15 @@ extern "C" int si_kv_unpack_flat(const int8_t* code, const int32_t* slot,
   const bool vec = group % 4 == 0 &&
                    ((reinterpret_cast<uintptr_t>(out_k) | reinterpret_cast<uintptr_t>(out_v)) & 15) == 0;
   const bool small = B * H * S < ((int64_t)1 << 31) && B < ((int64_t)1 << 31);
-  // Rows of fewer than 4 or more than 1024 values, and groups that straddle four
-  // of them, go to the token-order kernels.
-  if (!(vec && small && D % 4 == 0 && D <= 1024))
+  // Groups that straddle four values go to the token-order kernels, and so do rows
+  // that are no whole 64 bytes of output (bucket order scatters them, and a line is
+  // then written in two pieces) or longer than 192 values (a token-order block
+  // covers as few rows). us in token and in bucket order, S = 8192, H = 32, every
+  // precision: D = 20 14.9 and 34.0, 32 21.8 and 16.3, 40 28.5 and 44.4, 80 48.6 and
+  // 43.9, 88 53.4 and 74.2, 112 62.8 and 60.1; with S * D as at D = 128: D = 192 65.7
+  // and 64.8, 256 51.7 and 61.7, 512 51.7 and 61.8. 25% fp16, 50% int8, 25% int4: D =
+  // 80 48.3 and 37.0, 192 67.0 and 54.1, 256 55.0 and 53.7.
+  if (!(vec && small && D % 16 == 0 && D <= 192))
     return si_kv_unpack(code, slot, buckets, scale_dtype, B, H, S, D, group, out_k, out_v, stream);
   const Buckets bk = to_buckets(buckets);
   // Rows per thread (U) and threads per block (NT) of the bucket-order pack and

@@ -530,10 +530,12 @@ def test_token_and_bucket_order_copies_agree(dev, dtype, shape):
     (2, 3, 37, 80, 16), (1, 5, 130, 96, 16), (1, 2, 40, 8, 16), (1, 3, 33, 24, 16),
     (2, 2, 21, 40, 8), (1, 2, 19, 104, 16), (3, 1, 17, 160, 32), (1, 2, 9, 248, 16),
     (1, 3, 11, 12, 16), (2, 2, 13, 20, 4), (1, 1, 5, 504, 8),
+    (1, 3, 29, 16, 16), (2, 2, 15, 192, 16), (1, 2, 13, 208, 16),
 ])
 def test_rows_of_any_chunk_count_bit_exact(dev, dtype, B, H, S, D, g):
     """Head dims that are no power of two of 16-byte chunks (bucket-order pack with
-    idle lanes, bucket-order unpack at any multiple of 4), int4 groups of a
+    idle lanes), both unpack orders at the edges of their rule (bucket order for
+    multiples of 16 up to 192), int4 groups of a
     power of two of chunks and of the whole row, through reuse and evict:
     every byte equal to the oracle's."""
     k, v = kv_inputs(B, H, S, D, dtype, seed=B * 1000 + S * 10 + D)
