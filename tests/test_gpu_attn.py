@@ -20,6 +20,20 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-3
 
 
+# Kernel and key parts by size (0), the 256-query kernel (-1), the
+# wave-per-half-tile kernel (1), the 256-query kernel with its keys in two parts.
+KERNELS = [0, -1, 1, 64 + 2]
+
+
+@pytest.fixture
+def attn_parts():
+    """Sets si_tune_attn_parts for one test."""
+    lib = _native.load()
+    yield lib.si_tune_attn_parts
+    lib.si_tune_attn_parts(0)
+    lib.si_tune_attn_offset64(0)
+
+
 def _rel_l2(a, b):
     a = torch.as_tensor(a).double()
     b = torch.as_tensor(b).double()
@@ -32,10 +46,12 @@ def _pack(k, v, codes, dev, group_size=16):
                               plan=plan)["packed_kv"]
 
 
+@pytest.mark.parametrize("parts", KERNELS)
 @pytest.mark.parametrize("qdtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,Sq,Skv,D", [(1, 2, 128, 64, 128), (2, 2, 100, 200, 128),
                                           (1, 3, 130, 257, 64), (1, 1, 1, 1, 64)])
-def test_attention_small_vs_oracle(dev, qdtype, B, H, Sq, Skv, D):
+def test_attention_small_vs_oracle(dev, attn_parts, parts, qdtype, B, H, Sq, Skv, D):
+    attn_parts(parts)
     k, v = kv_inputs(B, H, Skv, D, torch.bfloat16, seed=Skv + D, outlier_frac=0.02)
     codes = mixed_codes(Skv, H, seed=Skv, probs=(1, 1, 2, 1), sink=min(4, Skv), evicted=0.05)
     cache = _pack(k, v, codes, dev)
@@ -167,11 +183,15 @@ def test_attention_entry_points_agree(dev, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("parts", KERNELS)
 @pytest.mark.parametrize("D", [64, 128])
-def test_attention_offset_widths_agree(dev, D):
+def test_attention_offset_widths_agree(dev, attn_parts, parts, D):
     """Caches below 2^31 bytes address bucket rows with 32-bit offsets; larger
     ones with 64-bit addresses. si_tune_attn_offset64 selects the 64-bit path at
-    any size: both give the same bits, and both match the oracle."""
+    any size: both give the same bits in each kernel, and both match the oracle.
+    (The 256-query kernel is not split with 64-bit addresses: its two parts
+    become the whole kernel.)"""
+    attn_parts(parts)
     B, H, S = 2, 3, 300
     k, v = kv_inputs(B, H, S, D, torch.bfloat16, seed=D + 7, outlier_frac=0.02)
     codes = mixed_codes(S, H, seed=D + 7, probs=(1, 1, 2, 1), sink=4, evicted=0.05)
@@ -180,11 +200,14 @@ def test_attention_offset_widths_agree(dev, D):
     q = torch.randn(B, H, S, D, generator=g).to(torch.bfloat16).to(dev)
     narrow = packed_attention(q, cache)
     lib = _native.load()
+    if parts > 64:
+        attn_parts(-1)
+        whole = packed_attention(q, cache)
+        assert not torch.equal(narrow, whole) and _rel_l2(narrow, whole) <= TOL
+        narrow = whole
+        attn_parts(parts)
     lib.si_tune_attn_offset64(1)
-    try:
-        wide = packed_attention(q, cache)
-    finally:
-        lib.si_tune_attn_offset64(0)
+    wide = packed_attention(q, cache)
     assert torch.equal(narrow, wide)
     rk, rv = O.kv_unpack(oracle_pack(k, v, codes))
     ref = O.attention(q.float().cpu().numpy().reshape(B * H, S, D), rk.reshape(B * H, S, D),
@@ -193,10 +216,12 @@ def test_attention_offset_widths_agree(dev, D):
 
 
 @pytest.mark.gpu
-def test_attention_extreme_scales(dev):
+@pytest.mark.parametrize("parts", KERNELS)
+def test_attention_extreme_scales(dev, attn_parts, parts):
     """Rows whose int8/int4 scales leave the range where a packed fp16 multiply
     rounds like the fp32 product (scales below 2^-14, or q * s near the fp16
     limit) take the decode's fp32 route; the result still matches the oracle."""
+    attn_parts(parts)
     B, H, S, D = 1, 2, 256, 128
     k, v = kv_inputs(B, H, S, D, torch.bfloat16, seed=5)
     k, v = k.float(), v.float()
