@@ -43,18 +43,35 @@ def test_plan_from_codes_matches_oracle(dev, S, H):
     assert plan.fingerprint == ref["fingerprint"]
 
 
-@pytest.mark.parametrize("S,H", [(1, 1), (7, 3), (1000, 3), (8192, 32), (40000, 32)])
+def _scan_on_the_host(codes, mask, S, H):
+    """Codes, slots, counts and lists of a plan scan: unknown and masked entries
+    are absent (4), slots count the entries of a code in order, lists hold h*S + t."""
+    code = np.where((codes < 0) | (codes > 3) | (mask != 0), 4, codes).astype(np.int8)
+    slot = np.full(code.size, -1, np.int32)
+    entry = np.arange(code.size, dtype=np.int64)
+    flat = entry % H * S + entry // H
+    lists = []
+    for p in range(4):
+        at = code == p
+        slot[at] = np.arange(at.sum(), dtype=np.int32)
+        lists.append(flat[at])
+    return code, slot, np.bincount(code, minlength=5).astype(np.int64), lists
+
+
+@pytest.mark.parametrize("S,H", [(1, 1), (7, 3), (1000, 3), (8192, 32), (32768, 32), (40000, 32)])
 def test_plan_scan_lists_matches_scan_then_scatter(dev, S, H):
-    """The evict rescan with its flat lists in one pass (si_plan_scan_lists)
-    gives the code / slot / counts of si_plan_scan and the lists of
-    si_plan_scatter, on the fused path and (40000 x 32: above 2^20 entries)
+    """The plan scan (si_plan_scan, then si_plan_scatter) and the evict rescan with
+    its flat lists in one pass (si_plan_scan_lists) give the host's codes, slots,
+    counts and lists, on the two-launch path and (40000 x 32: above 2^20 entries)
     on the three-pass fallback; no list is written at or past its capacity."""
     from shadowinfer_amd import _native
     import ctypes
     rng = np.random.default_rng(S + H)
-    codes = torch.from_numpy(rng.integers(-1, 6, size=S * H).astype(np.int8)).to(dev)
-    mask = torch.from_numpy((rng.random(S * H) < 0.3).astype(np.uint8)).to(dev)
+    host_codes = rng.integers(-1, 6, size=S * H).astype(np.int8)
+    host_mask = (rng.random(S * H) < 0.3).astype(np.uint8)
+    codes, mask = torch.from_numpy(host_codes).to(dev), torch.from_numpy(host_mask).to(dev)
     n = S * H
+    want_code, want_slot, want_counts, want_lists = _scan_on_the_host(host_codes, host_mask, S, H)
     sp = _native.stream(dev)
     ws_b = _native.size_query("si_plan_workspace_bytes", n)
     ws = torch.empty(ws_b, dtype=torch.uint8, device=dev)
@@ -63,10 +80,15 @@ def test_plan_scan_lists_matches_scan_then_scatter(dev, S, H):
     cnt0 = torch.empty(5, dtype=torch.int64, device=dev)
     _native.call("si_plan_scan", codes.data_ptr(), mask.data_ptr(), n, code0.data_ptr(),
                  slot0.data_ptr(), cnt0.data_ptr(), ws.data_ptr(), ws_b, sp)
-    counts = [int(c) for c in cnt0.tolist()]
+    counts = [int(c) for c in want_counts]
+    assert cnt0.tolist() == counts
+    np.testing.assert_array_equal(code0.cpu().numpy(), want_code)
+    np.testing.assert_array_equal(slot0.cpu().numpy(), want_slot)
     ref = [torch.empty(counts[p], dtype=torch.long, device=dev) for p in range(4)]
     _native.call("si_plan_scatter", code0.data_ptr(), slot0.data_ptr(), S, H,
                  _native.table4([r.data_ptr() for r in ref]), _native.table4([None] * 4), sp)
+    for p in range(4):
+        np.testing.assert_array_equal(ref[p].cpu().numpy(), want_lists[p])
     # lists one row short of the new sizes, inside buffers with a sentinel tail
     cap = [max(c - 1, 0) for c in counts[:4]]
     bufs = [torch.full((c + 8,), -7, dtype=torch.long, device=dev) for c in cap]
