@@ -803,10 +803,11 @@ def test_rope_pack_support_rule():
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("M,V", [(3, 2034), (3, 2035), (2, 8190), (5, 16379), (4, 32754), (4, 32755),
-                                 (3, 32769), (7, 13)])
+                                 (3, 32769), (7, 13), (3, 32768), (3, 32776), (2, 50000)])
 def test_argmax_conf_row_lengths(dev, dtype, M, V):
-    """Row lengths at both sides of each register-held size and rows that start
-    between 16-byte boundaries (odd V), each row with its maximum in the first or
+    """Row lengths at both sides of each register-held size, longer ones in eights
+    (32776, 50000) and one by one (32769), and rows that start between 16-byte
+    boundaries (odd V), each row with its maximum in the first or
     last column and the neighbouring rows' columns larger: tokens and confidences
     as torch's softmax + max on the GPU, outside the oracle's flagged rows."""
     from shadowinfer_amd.execution import argmax_confidence
