@@ -16,7 +16,7 @@ __device__ __forceinline__ float wave_amax(float m) {
   return m;
 }
 
-// Block-wide |max| for a 256-thread block (4 waves).
+// Block-wide |max| for a block of NW waves.
 template <int NW = 4>
 __device__ __forceinline__ float block_amax(float m, float* lds) {
   m = wave_amax(m);

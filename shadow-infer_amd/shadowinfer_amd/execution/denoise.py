@@ -169,9 +169,9 @@ class PackedDiffusionLlama:
             q, k, v = row_ops.rope_split(qkv, cos, sin, B, S, H, D)
             cache = PackedKVCache.pack(k, v, None, group_size=c.int4_group_size,
                                        plan=plan)["packed_kv"]
-        # one attention kernel at every length: a row rounded otherwise flips int4
-        # codes of the next layer's cache, which shows in the logits (4% after two
-        # layers), so splitting the keys would make a trajectory depend on the shape
+        # the whole kernel: split keys round P at other maxima, with the same error,
+        # but int8 activations and int4 codes of the layers behind flip with it (3.8%
+        # of the logits' norm after two layers), and a step keeps the results it had
         attn = packed_attention(q, cache, out_dtype=self.dtype, token_major=True,
                                 split_keys=False)
         o = F.linear(attn.view(T, Hd), L.w_o)
