@@ -690,11 +690,13 @@ __global__ __launch_bounds__(512) void attn_packed_fwd(
     int sl4[4] = {sl.x, sl.y, sl.z, sl.w};
     if constexpr (P == SI_PREC_FP32) return;  // read at decode time
     // Keys past the tile's valid count (only in a phase's last tile: nv is
-    // wave-uniform) read row 0 of the same (non-empty) bucket: their list
-    // entries are not written, and their scores are masked to -inf.
+    // wave-uniform) read the row of the tile's first key: their list entries are not
+    // written, and their scores are masked to -inf. A row of another head would not
+    // do: where one of its values is infinite in fp16, P = 0 does not cancel it.
     if (nv < BN) {
+      const int own = lh[(int64_t)tt * BN];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sl4[i] = 4 * kg + i < nv ? sl4[i] : 0;
+      for (int i = 0; i < 4; ++i) sl4[i] = 4 * kg + i < nv ? sl4[i] : own;
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

@@ -350,7 +350,8 @@ def test_attention_key_parts_match_oracle(dev, parts, B, H, Sq, S, D, dtype, g, 
 @pytest.mark.parametrize("dtype,code,parts", [
     (torch.float32, 0, -1), (torch.float32, 0, 1), (torch.float32, 0, 3), (torch.float32, 0, 64 + 2),
     (torch.bfloat16, 0, 2), (torch.bfloat16, 1, 1), (torch.bfloat16, 2, 2), (torch.bfloat16, 3, 1),
-    (torch.float32, 2, 1), (torch.float32, 3, 2)])
+    (torch.float32, 2, 1), (torch.float32, 3, 2),
+    (torch.bfloat16, 1, -1), (torch.bfloat16, 2, -1), (torch.bfloat16, 3, 64 + 2), (torch.float32, 2, -1)])
 @pytest.mark.parametrize("D", [64, 128])
 def test_attention_values_past_fp16_stay_in_their_head(dev, D, dtype, code, parts):
     """Head 0's first value row is 1e5, infinite as an fp16 operand; the other
