@@ -377,8 +377,8 @@ __global__ __launch_bounds__(256) void swiglu_quant(const void* __restrict__ gu,
 // (row_argmax_conf_regs): one read of the logits instead of three passes of
 // which the later two came from L2. The kernel is bound by its VALU work on
 // every logit, so no pass looks for NaN or infinities (a row that holds one, or
-// only -inf, has a NaN sum) and the sum takes expf's bits from row_exp: 10
-// instructions for 15, 2048 rows of 32000 bf16 logits 38 us against 43 with expf
+// only -inf, has a NaN sum) and the sum takes expf's bits from add_exp: 11
+// instructions for 16, 2048 rows of 32000 bf16 logits 38 us against 43 with expf
 // itself (33 with exp2 of a rounded d * log2(e), up to 45 ulp off: not kept).
 // 2048 rows of 32000 bf16 65 -> 38 us (131 MB: 26 us at the copy rate), of 32001
 // fp16 138 -> 40, of 32000 fp32 113 -> 59, 8 rows of 32000 bf16 20 -> 12.
@@ -398,12 +398,17 @@ __device__ __forceinline__ void for_row(const void* __restrict__ logits, int64_t
   }
 }
 
-// exp(d) for d <= 0 (NaN stays NaN): d * log2(e) as an exact product h + l, the
-// nearest integer e of h, 2^(h - e + l) on v_exp_f32 and e added to its exponent.
+// s + exp(d) for d <= 0 (NaN, with any payload, stays NaN): d * log2(e) as an exact
+// product h + l, the nearest integer e of h, 2^(h - e + l) on v_exp_f32, and 2^e by
+// the exact product of the addition's fma. fp16 logits add e to the exponent
+// instead, which would end the NaN of a payload in its low 9 bits (theirs are 0): the
+// compiler schedules their conversions better around it (2048 x 32000 39.7 us for
+// 42.3; bf16 38.3 in both).
 // Of all floats from -87 to 0, all but 16 give expf's bits, and the largest error is
-// expf's (0.857 ulp; mean 0.257 in both). Below -87 it gives exp(-87) = 1.6e-38
-// where expf falls to 0: the sum it goes into holds expf(0) = 1.
-__device__ __forceinline__ float row_exp(float d) {
+// expf's (0.857 ulp; mean 0.257 in both). Below -87 it adds exp(-87) = 1.6e-38
+// where expf falls to 0: the sum holds expf(0) = 1.
+template <int DT>
+__device__ __forceinline__ float add_exp(float s, float d) {
   constexpr float kHi = 1.44269502f, kLo = 1.92596303e-8f;  // log2(e)
   constexpr float kRound = 12582912.0f;                     // 1.5 * 2^23
   d = __builtin_elementwise_maximum(d, -87.0f);
@@ -411,7 +416,9 @@ __device__ __forceinline__ float row_exp(float d) {
   const float l = __builtin_fmaf(d, kLo, __builtin_fmaf(d, kHi, -h));
   const float t = h + kRound, e = t - kRound;
   const float r = __builtin_amdgcn_exp2f((h - e) + l);
-  return __uint_as_float(__float_as_uint(r) + (__float_as_uint(t) << 23));
+  const uint32_t k = __float_as_uint(t) << 23;
+  if constexpr (DT == SI_DT_F16) return s + __uint_as_float(__float_as_uint(r) + k);
+  return __builtin_fmaf(r, __uint_as_float(k + 0x3f800000u), s);
 }
 
 // The row's result from thread-wise first candidates (INT64_MAX: none).
@@ -454,7 +461,7 @@ __global__ __launch_bounds__(256) void row_argmax_conf(const void* __restrict__ 
     for_row<DT, VEC>(logits, m, V, [&](float x, int64_t) { mx = fmaxf(mx, x); });
     mx = block_max(mx, lds);
     float s = 0.0f;
-    for_row<DT, VEC>(logits, m, V, [&](float x, int64_t) { s += row_exp(x - mx); });
+    for_row<DT, VEC>(logits, m, V, [&](float x, int64_t) { s = add_exp<DT>(s, x - mx); });
     s = block_sum(s, lds);
     if (s != s) {
       store_nan_row(DT, m, tok, conf);
@@ -562,7 +569,7 @@ __global__ __launch_bounds__(256, R * (DT == SI_DT_F32 ? 8 : 4) > 64 ? 2 : 4) vo
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s += row_exp(value(w[r], e) - mx);
+      for (int e = 0; e < 8; ++e) s = add_exp<DT>(s, value(w[r], e) - mx);
     s = block_sum(s, lds);
     if (s != s) {
       store_nan_row(DT, m, tok, conf);

@@ -856,6 +856,26 @@ def test_confidence_sum_adds_the_library_exponential(dev, V):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,bits", [
+    (torch.float32, [0x7fc00000, 0x7fffffff, -1, 0x7fc00001, -0x3fff01, 0x7f800001, 0x7fc001fe]),
+    (torch.bfloat16, [0x7fc0, 0x7fff, -1, 0x7f81, 0x7fc1]),
+    (torch.float16, [0x7e00, 0x7fff, -1, 0x7c01, 0x7e01])])
+@pytest.mark.parametrize("V", [5, 2048, 32000, 32769, 40000])
+def test_argmax_conf_keeps_nan_of_any_payload(dev, V, dtype, bits):
+    """A NaN logit makes its row NaN (token 0) whatever its sign and payload, also
+    a signalling one; the rows beside it keep their results."""
+    from shadowinfer_amd.execution import argmax_confidence
+    x = torch.randn(2 * len(bits), V, generator=torch.Generator().manual_seed(V)).to(dtype)
+    clean = x.clone().to(dev)
+    for i, b in enumerate(bits):
+        x.view(torch.int32 if dtype == torch.float32 else torch.int16)[2 * i, (i * 7919) % V] = b
+    tok, conf = argmax_confidence(x.to(dev))
+    assert bool(torch.isnan(conf[::2]).all()) and tok[::2].tolist() == [0] * len(bits)
+    tok0, conf0 = argmax_confidence(clean)
+    assert torch.equal(tok[1::2], tok0[1::2]) and torch.equal(conf[1::2], conf0[1::2])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W", [1, 63, 1024, 1025, 3000])
 def test_schedule_rows_nan_ties_and_signs(dev, W):
     """The unmasking rule with NaN confidences (largest for the fallback, NaN kept
